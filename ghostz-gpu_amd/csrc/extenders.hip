@@ -28,6 +28,7 @@
 #include "gz_device.h"
 #include "gz_runtime.h"
 #include "gz_scan.h"
+#include "wave_dp.h"
 
 namespace gz {
 
@@ -496,13 +497,14 @@ constexpr int kGappedBlock = 64;
 
 // Jobs [begin, end) (through `order` when set: slot k runs job order[k],
 // which must be below `limit`), or the `*list_count` jobs of `list` when
-// list is set; a job whose band outgrows the W-column ring is appended to
+// list is set and they are more than list_over; a job whose band outgrows the W-column ring is appended to
 // the overflow list for the next, wider ring.  Results land at each job's
 // own index.
 template <bool kReverse, int W, bool kShort>
 __global__ void __launch_bounds__(kGappedBlock)
     GappedKernel(size_t begin, size_t end, const uint32_t *list, const uint32_t *list_count,
-                 const uint32_t *order, size_t limit, GappedParams P, const int *matrix,
+                 uint32_t list_over, const uint32_t *order, size_t limit, GappedParams P,
+                 const int *matrix,
                  uint32_t nl, uint32_t *qpos, uint32_t *dpos, int *scores, uint32_t *cells,
                  uint32_t *overflow_count, uint32_t *overflow_list, uint32_t *failed) {
   using Ring = typename std::conditional<kShort, LaneRingLds16, LaneRingLds>::type;
@@ -518,6 +520,7 @@ __global__ void __launch_bounds__(kGappedBlock)
   R.mask = W - 1;
   R.lane = threadIdx.x;
   const size_t n = list ? (size_t)*list_count : end - begin;
+  if (list && n <= list_over) return;
   for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
        k += (size_t)gridDim.x * blockDim.x) {
     const size_t i = list ? (size_t)list[k] : order ? (size_t)order[begin + k] : begin + k;
@@ -1254,11 +1257,12 @@ struct gz_gapped_extender_s {
   // ring's overflow skips the 64-column ring); GZ_GAPPED_WAVE=never|direct
   int wave_mode = kWaveAuto;
   // workspace
-  // [0] jobs out of the narrow ring, [1] failures, [2] jobs out of the
-  // 64-column ring, [3] the work queue's head
+  // [0] jobs out of the narrow ring, [1] failures, [2] jobs of the row
+  // kernel past 64 columns, [3] the work queue's head, [4] jobs of the second
+  // overflow list, [5] the row kernel's queue head over the first
   uint32_t *counters = nullptr;
   uint32_t *overflow_list = nullptr;   // out of the narrow ring
-  uint32_t *overflow_list2 = nullptr;  // out of the 64-column ring
+  uint32_t *overflow_list2 = nullptr;  // for the global ring
   size_t overflow_capacity = 0;
   int2 *wide_cells = nullptr;
   uint8_t *wide_codes = nullptr;
@@ -1335,9 +1339,8 @@ gz_status gz_gapped_extender_convert_to_gapped_extension_seeds_async(
 }
 
 extern "C++" {
-// Device memory one gapped run uses beyond its jobs: counters ([0] jobs out
-// of the narrow ring, [1] failures, [2] jobs out of the 64-column ring), the
-// two overflow lists (room for every job) and the global ring (kWideSlots
+// Device memory one gapped run uses beyond its jobs: the counters (as in the
+// handle), the two overflow lists (room for every job) and the global ring (kWideSlots
 // slots of `wide` cells and codes).
 struct GappedWork {
   uint32_t *counters;
@@ -1353,6 +1356,23 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
                          size_t size, size_t wide_first, const uint32_t *order, uint32_t *d_q,
                          uint32_t *d_d, int *d_scores, uint32_t *d_cells, hipStream_t s) {
   uint32_t *narrow_out = w.counters, *failures = w.counters + 1, *wide_out = w.counters + 2;
+  uint32_t *list2_out = w.counters + 4;
+  // one wave per job with the row in registers (wave_dp.h), for calls with
+  // few jobs and for the bands that outgrow the first ring
+  const bool rows = h->wave_mode == kWaveAuto && WaveDpServes(P.cutoff, P.gap_open, P.gap_ext);
+  const WaveDpParams R = {P.queries, P.database, P.delim, P.gap_open + P.gap_ext,
+                          P.gap_ext, P.cutoff};
+  const uint32_t *none = nullptr;
+#define GZ_ROWS(N, LIST, COUNT, ORDER, HEAD, NARROW)                                            \
+  {                                                                                             \
+    const WaveDpGrid g = WaveDpGridFor(N);                                                      \
+    hipLaunchKernelGGL((GappedRowKernel<kReverse>), dim3(g.blocks), dim3(kWaveDpBlock), 0, s,    \
+                       (uint32_t)(N), LIST, COUNT, ORDER, (uint32_t)size, g.batch, HEAD, R,      \
+                       h->matrix, h->number_letters, d_q, d_d, d_scores, d_cells, list2_out,     \
+                       w.overflow_list2, (int)h->narrow, NARROW, wide_out, failures);            \
+  }
+  const bool row_jobs = rows && size <= kWaveDpJobs;
+  if (row_jobs) GZ_ROWS(size, none, none, order, w.counters + 3, narrow_out)
   // 16-bit cells in the LDS rings when the cutoff and gap costs allow them
   // (LaneRingLds16); bands whose scores grow past them move on like bands
   // that outgrow the ring
@@ -1363,14 +1383,17 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
 #define GZ_RING64(SHORT, GRID, BEGIN, END, LIST, COUNT, ORDER)                                 \
   hipLaunchKernelGGL((GappedKernel<kReverse, kGappedRing, SHORT>), GRID, dim3(kGappedBlock), 0, \
                      s, (size_t)(BEGIN), (size_t)(END), (const uint32_t *)(LIST),              \
-                     (const uint32_t *)(COUNT), ORDER, size, P, h->matrix, h->number_letters,  \
-                     d_q, d_d, d_scores, d_cells, wide_out, w.overflow_list2, failures)
-  if (wide_first > 0) {
+                     (const uint32_t *)(COUNT), rows ? kWaveDpJobs : 0u, ORDER, size, P,       \
+                     h->matrix, h->number_letters,                                             \
+                     d_q, d_d, d_scores, d_cells, list2_out, w.overflow_list2, failures)
+  if (!row_jobs && wide_first > 0) {
     const dim3 grid(GridFor(wide_first, kGappedBlock, 256u * 32));
     if (short_cells) GZ_RING64(true, grid, 0, wide_first, nullptr, nullptr, order);
     else GZ_RING64(false, grid, 0, wide_first, nullptr, nullptr, order);
   }
-  if (size > wide_first && h->persistent && wide_first == 0) {
+  if (row_jobs) {
+    // every job has run
+  } else if (size > wide_first && h->persistent && wide_first == 0) {
     // one persistent launch over every job, sized to the waves the device
     // holds at once
 #define GZ_QUEUE(WIDTH, SHORT)                                                               \
@@ -1397,7 +1420,7 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
 #define GZ_NARROW(WIDTH, SHORT)                                                              \
   hipLaunchKernelGGL((GappedKernel<kReverse, WIDTH, SHORT>), grid, dim3(kGappedBlock), 0, s, \
                      wide_first, size, (const uint32_t *)nullptr, (const uint32_t *)nullptr, \
-                     order, size, P, h->matrix, h->number_letters, d_q, d_d, d_scores,       \
+                     0u, order, size, P, h->matrix, h->number_letters, d_q, d_d, d_scores,       \
                      d_cells, narrow_out, w.overflow_list, failures)
     if (h->narrow == 16) {
       if (short_cells) GZ_NARROW(16, true);
@@ -1419,21 +1442,26 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
     hipLaunchKernelGGL((GappedWaveKernel<kReverse>), wave_grid, dim3(kWave), 0, s, P, h->matrix,
                        h->number_letters, d_q, d_d, d_scores, d_cells, narrow_out,
                        w.overflow_list, w.wide_cells, w.wide, failures);
-  } else {
-    // the narrow ring's overflow; 16-bit cells leave LDS for more blocks
-    const uint32_t *none = nullptr;
+  } else if (!row_jobs) {
+    // the narrow ring's overflow: one wave per job while the waves are
+    // enough for the list, else the 64-column ring (each looks at the
+    // count); 16-bit cells leave LDS for more blocks
+    if (rows)
+      GZ_ROWS(std::min<size_t>(size, kWaveDpJobs), w.overflow_list, narrow_out, none,
+              w.counters + 5, (uint32_t *)nullptr)
     if (short_cells) GZ_RING64(true, dim3(256u * 6), 0, 0, w.overflow_list, narrow_out, none);
     else GZ_RING64(false, dim3(256u * 4), 0, 0, w.overflow_list, narrow_out, none);
   }
 #undef GZ_RING64
+#undef GZ_ROWS
   if (wave)
     hipLaunchKernelGGL((GappedWaveKernel<kReverse>), wave_grid, dim3(kWave), 0, s, P, h->matrix,
-                       h->number_letters, d_q, d_d, d_scores, d_cells, wide_out,
+                       h->number_letters, d_q, d_d, d_scores, d_cells, list2_out,
                        w.overflow_list2, w.wide_cells, w.wide, failures);
   else
     hipLaunchKernelGGL((GappedWideKernel<kReverse>), dim3(w.wide_slots / kGappedBlock),
                        dim3(kGappedBlock), 0, s, P, h->matrix, h->number_letters, d_q, d_d,
-                       d_scores, d_cells, wide_out, w.overflow_list2, w.wide_cells,
+                       d_scores, d_cells, list2_out, w.overflow_list2, w.wide_cells,
                        w.wide_codes, w.wide, failures);
 }
 }  // extern "C++"
@@ -1459,14 +1487,14 @@ static gz_status GappedLaunchAll(gz_gapped_extender_t h, const GappedWork &w, si
 // the queue head are zeroed, the failure count ([1]) is kept until read.  A
 // kernel, not a memset, so that the sequence can be captured in a graph.
 __global__ void ResetRunCountersKernel(uint32_t *counters, int all) {
-  if (threadIdx.x < 4 && (all || threadIdx.x != 1)) counters[threadIdx.x] = 0;
+  if (threadIdx.x < 8 && (all || threadIdx.x != 1)) counters[threadIdx.x] = 0;
 }
 
 // Allocates the handle's workspace for runs of up to `size` jobs (no-op
 // when it is large enough).
 static gz_status GappedReserve(gz_gapped_extender_t h, size_t size, hipStream_t s) {
   if (!h->counters) {
-    GZ_HIP_CHECK(gz::Malloc(&h->counters, 4 * sizeof(uint32_t)));
+    GZ_HIP_CHECK(gz::Malloc(&h->counters, 8 * sizeof(uint32_t)));
     hipLaunchKernelGGL(ResetRunCountersKernel, dim3(1), dim3(64), 0, s, h->counters, 1);
     GZ_HIP_CHECK(hipGetLastError());
   }
@@ -1480,8 +1508,12 @@ static gz_status GappedReserve(gz_gapped_extender_t h, size_t size, hipStream_t 
     GZ_HIP_CHECK(gz::Malloc(&h->overflow_list2, cap * sizeof(uint32_t)));
     h->overflow_capacity = cap;
   }
-  // lanes: one per job at most, at least kWideSlots, within the budget
-  const size_t by_jobs = (size + 63) / 64 * 64;
+  // lanes: one per job at most, at least kWideSlots, within the budget; a
+  // call that runs on the row kernel leaves the global ring next to nothing
+  // (bands past 128 columns)
+  const bool rows = h->wave_mode == kWaveAuto && size <= kWaveDpJobs &&
+                    WaveDpServes(h->cutoff, h->gap_open, h->gap_ext);
+  const size_t by_jobs = rows ? 0 : (size + 63) / 64 * 64;
   const uint32_t want = (uint32_t)std::max<size_t>(
       kWideSlots, std::min<size_t>(WideSlotsFor(h->wide), by_jobs));
   if (h->wide_allocated < h->wide || h->wide_slots < want) {
@@ -1601,7 +1633,7 @@ gz_status ScratchOfCurrentDevice(uint8_t **out) {
 }
 
 __global__ void ClearCountersKernel(uint32_t *counters) {
-  if (threadIdx.x < 4) counters[threadIdx.x] = 0;
+  if (threadIdx.x < 8) counters[threadIdx.x] = 0;
 }
 
 }  // namespace
@@ -1676,10 +1708,10 @@ gz_status gz_gapped_extender_overflows(gz_gapped_extender_t h, uint32_t *narrow,
   GZ_REQUIRE(h && narrow && ring64, "null argument");
   *narrow = *ring64 = 0;
   if (h->counters) {
-    uint32_t c[3];
+    uint32_t c[5];
     GZ_HIP_CHECK(hipMemcpy(c, h->counters, sizeof(c), hipMemcpyDeviceToHost));
     *narrow = c[0];
-    *ring64 = c[2];
+    *ring64 = std::max(c[2], c[4]);
   }
   return GZ_OK;
 }
