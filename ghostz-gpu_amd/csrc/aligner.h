@@ -24,6 +24,7 @@
 #include "results.h"
 #include "query_lists_device.h"
 #include "search_device.h"
+#include "traceback.h"
 
 struct gz_gapped_extender_s;
 
@@ -132,9 +133,6 @@ class Aligner : public PresearchDevice {
   size_t lookup_chunk_ = kNoChunk;  // database chunk of the seed stage's lookup
   std::vector<void *> query_buffers_;
   unsigned seed_kinds_ = 3;
-  // timing events: [0, 2) the gapped kernels', [4, 6) the result build's
-  // (the stages may run on different host threads)
-  hipEvent_t ev_[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   // The gapped stage's two pipeline slots: GappedPrepare uploads a slot's
   // jobs and orders them on the schedule stream, GappedRun extends them on
   // the extension stream once the slot's `ready` event has passed, so one
@@ -159,9 +157,7 @@ class Aligner : public PresearchDevice {
   bool two_extensions_ = false;
   hipEvent_t run_ev_[2][2] = {};  // per slot: around its gapped kernels
   std::mutex stats_mutex_;        // AlignStats updates from both slots
-  // result-build workspace
-  void *tb_ws_ = nullptr;
-  size_t tb_ws_cap_ = 0;
+  TracebackRunner tracebacks_;    // the result build's
   uint32_t max_query_length_ = 0;
   // pinned job buffers per pipeline slot
   std::vector<std::pair<void *, size_t> > pinned_jobs_;

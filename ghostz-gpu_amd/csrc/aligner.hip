@@ -91,11 +91,8 @@ Aligner::~Aligner() {
     for (hipEvent_t e : {S.ready, S.ev_begin, S.ev_end})
       if (e) (void)hipEventDestroy(e);
   }
-  if (tb_ws_) (void)gz::Free(tb_ws_);
   for (auto &b : pinned_jobs_)
     if (b.first) (void)gz::HostFree(b.first);
-  for (hipEvent_t e : ev_)
-    if (e) (void)hipEventDestroy(e);
   for (auto &slot : tune_ev_)
     for (hipEvent_t e : slot)
       if (e) (void)hipEventDestroy(e);
@@ -583,52 +580,14 @@ int Aligner::Tracebacks(size_t ci, const std::vector<TracebackJob> &jobs, int cu
   const size_t n = jobs.size();
   out->resize(n);
   if (n == 0) return 0;
-  hipStream_t s = traceback_stream_;
-  for (int i = 4; i < 6; ++i)
-    if (!ev_[i]) GZ_TRY(hipEventCreate(&ev_[i]));
-  // m jobs with the given per-lane capacities: lanes resident at once (up
-  // to seven 64-lane blocks per CU), bounded by a 12 GB scratch budget
-  auto pass = [&](const TracebackJob *hjobs, size_t m, const LaneCaps &caps,
-                  TracebackOut *hout) -> hipError_t {
-    const size_t budget = (size_t)12 << 30;
-    size_t lanes = std::min<size_t>((m + 63) / 64 * 64, (size_t)7 * 64 * 256);
-    lanes = std::max<size_t>(64, std::min(lanes, budget / caps.bytes_per_lane / 64 * 64));
-    const size_t a_jobs = AlignUp(m * sizeof(TracebackJob), 256);
-    const size_t a_outs = AlignUp(m * sizeof(TracebackOut), 256);
-    const size_t bytes = a_jobs + a_outs + lanes * caps.bytes_per_lane;
-    if (tb_ws_cap_ < bytes) {
-      if (tb_ws_) (void)gz::Free(tb_ws_);
-      tb_ws_ = nullptr;
-      tb_ws_cap_ = 0;
-      const hipError_t a = gz::Malloc(&tb_ws_, bytes);
-      if (a != hipSuccess) return a;
-      tb_ws_cap_ = bytes;
-    }
-    TracebackJob *d_jobs = (TracebackJob *)tb_ws_;
-    TracebackOut *d_outs = (TracebackOut *)((char *)tb_ws_ + a_jobs);
-    uint8_t *scratch = (uint8_t *)tb_ws_ + a_jobs + a_outs;
-    hipError_t e = hipMemcpyAsync(d_jobs, hjobs, m * sizeof(TracebackJob),
-                                  hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipEventRecord(ev_[4], s);
-    if (e == hipSuccess)
-      e = TracebackLaunch(dq_.packed, chunks_[ci]->packed, d_jobs, (uint32_t)m, d_matrix_,
-                          opt_.search.nl, opt_.search.gap_open, opt_.search.gap_extension,
-                          cutoff, scratch, caps, (uint32_t)lanes, d_outs, s);
-    if (e == hipSuccess) e = hipEventRecord(ev_[5], s);
-    // the outputs' copy is queued once the kernel is done (as in GappedRun)
-    if (e == hipSuccess) e = hipEventSynchronize(ev_[5]);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(hout, d_outs, m * sizeof(TracebackOut), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    float ms = 0;
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms, ev_[4], ev_[5]);
-    if (e == hipSuccess) st->traceback_kernel_ms += ms;
-    return e;
-  };
-  const LaneCaps caps = TracebackCaps(max_query_length_, db_->max_length);
-  GZ_TRY(pass(jobs.data(), n, caps, out->data()));
-  // results whose op rows outgrow the lane's arena are rebuilt on the host
-  // (on all threads): a long band on one lane runs far slower than on a core
+  const TracebackInputs in = {dq_.packed,        chunks_[ci]->packed,   max_query_length_,
+                              db_->max_length,   d_matrix_,             opt_.search.nl,
+                              opt_.search.gap_open, opt_.search.gap_extension, cutoff};
+  float ms = 0;
+  GZ_TRY(tracebacks_.Run(in, jobs.data(), (uint32_t)n, out->data(), traceback_stream_, &ms));
+  st->traceback_kernel_ms += ms;
+  // results whose op rows outgrow the arena are rebuilt on the host (on all
+  // threads): a long band on one lane runs far slower than on a core
   return 0;
 }
 

@@ -400,22 +400,11 @@ gz_status gz_build_results(const uint64_t *pq, const uint64_t *pd, const gz_trac
   GZ_REQUIRE(n < (1ull << 31), "gz_build_results: too many jobs");
   if (n == 0) return GZ_OK;
   hipStream_t s = stream ? stream->s : nullptr;
-  const LaneCaps caps = TracebackCaps(max_query_length, max_subject_length);
-  const size_t lanes = std::min<size_t>((n + 63) / 64 * 64, (size_t)1 << 14);
-  void *ws = nullptr;
-  const size_t a_jobs = AlignUp(n * sizeof(TracebackJob), 256);
-  const size_t a_outs = AlignUp(n * sizeof(TracebackOut), 256);
-  GZ_HIP_CHECK(gz::Malloc(&ws, a_jobs + a_outs + lanes * caps.bytes_per_lane));
-  hipError_t e = hipMemcpyAsync(ws, jobs, n * sizeof(TracebackJob), hipMemcpyHostToDevice, s);
-  if (e == hipSuccess)
-    e = TracebackLaunch(pq, pd, (const TracebackJob *)ws, (uint32_t)n, d_matrix, nl, gap_open,
-                        gap_ext, cutoff, (uint8_t *)ws + a_jobs + a_outs, caps, (uint32_t)lanes,
-                        (TracebackOut *)((char *)ws + a_jobs), s);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(results, (char *)ws + a_jobs, n * sizeof(TracebackOut),
-                       hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)gz::Free(ws);
+  const TracebackInputs in = {pq,       pd,      max_query_length, max_subject_length, d_matrix, nl,
+                              gap_open, gap_ext, cutoff};
+  TracebackRunner run;
+  const hipError_t e = run.Run(in, reinterpret_cast<const TracebackJob *>(jobs), (uint32_t)n,
+                               reinterpret_cast<TracebackOut *>(results), s, nullptr);
   GZ_HIP_CHECK(e);
   return GZ_OK;
 }

@@ -1361,7 +1361,7 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
   // few jobs and for the bands that outgrow the first ring
   const bool rows = h->wave_mode == kWaveAuto && WaveDpServes(P.cutoff, P.gap_open, P.gap_ext);
   const WaveDpParams R = {P.queries, P.database, P.delim, P.gap_open + P.gap_ext,
-                          P.gap_ext, P.cutoff};
+                          P.gap_ext, P.cutoff, kWaveDpMargin};
   const uint32_t *none = nullptr;
 #define GZ_ROWS(N, LIST, COUNT, ORDER, HEAD, NARROW)                                            \
   {                                                                                             \

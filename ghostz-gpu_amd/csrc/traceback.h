@@ -15,18 +15,39 @@ struct LaneCaps {
   size_t bytes_per_lane = 0;
 };
 
-// The op arena of a lane.
+// The op arena of a side, in bytes; a side whose rows need more is flagged.
 constexpr uint32_t kTracebackArena = 1u << 16;
 
-LaneCaps TracebackCaps(uint32_t max_query_length, uint32_t max_subject_length,
-                       uint32_t arena = kTracebackArena);
+// Packed sequences, score parameters and the bounds of the jobs: the longest
+// framed query, the longest subject.
+struct TracebackInputs {
+  const uint64_t *queries, *database;
+  uint32_t max_query_length, max_subject_length;
+  const int *matrix;  // on the device
+  uint32_t nl;
+  int gap_open, gap_ext, cutoff;
+};
 
-// One result per job; `lanes` (a multiple of 64) is the number of lanes the
-// scratch holds (lanes x caps.bytes_per_lane bytes).
-hipError_t TracebackLaunch(const uint64_t *packed_queries, const uint64_t *packed_database,
-                           const TracebackJob *jobs, uint32_t n, const int *matrix,
-                           uint32_t nl, int gap_open, int gap_ext, int cutoff,
-                           uint8_t *scratch, const LaneCaps &caps, uint32_t lanes,
-                           TracebackOut *outs, hipStream_t stream);
+// Runs jobs, one after the other call, in a workspace that it keeps.
+class TracebackRunner {
+ public:
+  TracebackRunner() = default;
+  ~TracebackRunner();
+  TracebackRunner(const TracebackRunner &) = delete;
+  TracebackRunner &operator=(const TracebackRunner &) = delete;
+  // jobs and outs on the host; synchronous.  kernel_ms (may be null): the
+  // kernels' time.
+  hipError_t Run(const TracebackInputs &in, const TracebackJob *jobs, uint32_t n,
+                 TracebackOut *outs, hipStream_t s, float *kernel_ms);
+
+ private:
+  static hipError_t Reserve(void **p, size_t *cap, size_t bytes);
+  // one lane per job (d_list: the n jobs to run)
+  hipError_t Lanes(const TracebackInputs &in, const TracebackJob *d_jobs, uint32_t n,
+                   const uint32_t *d_list, TracebackOut *d_outs, hipStream_t s);
+  void *ws_ = nullptr, *lane_ws_ = nullptr;
+  size_t cap_ = 0, lane_cap_ = 0;
+  hipEvent_t ev_[2] = {nullptr, nullptr};
+};
 
 }  // namespace gz

@@ -4,24 +4,29 @@
 // result cutoff and a traceback (GappedExtender::ExtendOneSide with
 // EditBlocks, src/gapped_extender.cpp:70-304,473-531), then counts length,
 // mismatches and gap openings / extensions over the joined edit script
-// (AlignerCommon::BuildResult, src/aligner_common.h:276-343).  One lane runs
-// one result.  The op store follows the reference's gap_states_ layout: rows
-// are laid back to back in one byte arena ([0] holds the first op, row r
+// (AlignerCommon::BuildResult, src/aligner_common.h:276-343).  One wave runs
+// one side of a result (TracebackWaveKernel: the DP of wave_dp.h with the
+// operations recorded); a lane runs a result where that form does not serve
+// (TracebackKernel).  The op store follows the reference's gap_states_ layout:
+// rows are laid back to back in one byte arena ([0] holds the first op, row r
 // starts where row r-1 ends), so the traceback's reads outside a row's band
 // see the same neighbouring bytes.  Cells an extension does not write hold a
 // marker; reading one (or reading outside the written range) means the
 // reference would have read a byte left by an earlier extension, and the
 // result is flagged so the host replays the chunk in the reference order.
-// Results whose scratch needs exceed the per-lane capacities are flagged for
-// the host as well.
+// Results whose op rows exceed the arena are flagged for the host as well.
 #include <hip/hip_runtime.h>
 
 #include <climits>
 
+#include <algorithm>
+
 #include "gz_common.h"
 #include "gz_device.h"
+#include "gz_runtime.h"
 #include "traceback.h"
 #include "ungapped.h"
+#include "wave_dp.h"
 
 namespace gz {
 
@@ -331,8 +336,9 @@ __device__ uint32_t Extend(const uint64_t *pq, int64_t q0, uint32_t s0len, const
 template <bool kShort>
 __global__ void __launch_bounds__(kTbThreads)
     TracebackKernel(const uint64_t *pq, const uint64_t *pd, const TracebackJob *jobs,
-                    uint32_t n, const int *matrix, uint32_t nl, int gap_open, int gap_ext,
-                    int cutoff, uint8_t *scratch, LaneCaps caps, TracebackOut *outs) {
+                    uint32_t n, const uint32_t *list, const int *matrix, uint32_t nl,
+                    int gap_open, int gap_ext, int cutoff, uint8_t *scratch, LaneCaps caps,
+                    TracebackOut *outs) {
   __shared__ int8_t sm[kTableDim * kTableDim];
   StageScoreTable(sm, matrix, nl);
   __syncthreads();
@@ -348,7 +354,8 @@ __global__ void __launch_bounds__(kTbThreads)
   L.row_cap = caps.rows;
   L.arena_cap = caps.arena;
   L.op_cap = caps.ops;
-  for (uint32_t j = lane_id; j < n; j += lanes) {
+  for (uint32_t k = lane_id; k < n; k += lanes) {
+    const uint32_t j = list ? list[k] : k;
     const TracebackJob job = jobs[j];
     TracebackOut o = {};
     Side rev, fwd;
@@ -399,34 +406,456 @@ __global__ void __launch_bounds__(kTbThreads)
   }
 }
 
-}  // namespace
+// ---------------------------------------------------------------------------
+// one wave per side
+// ---------------------------------------------------------------------------
+// What a side's wave leaves for its result.
+struct TracebackHalf {
+  int score;
+  uint32_t q, d;  // where the extension ends
+  uint32_t length, mismatches, gap_openings, gap_extensions;
+  uint32_t flags;  // kTracebackStale / Overflow / kNeedsLane
+};
+constexpr uint32_t kNeedsLane = 4;
 
-LaneCaps TracebackCaps(uint32_t max_query_length, uint32_t max_subject_length,
-                       uint32_t arena) {
+constexpr int kTbWaveBlock = 256;
+// Waves resident at once: four per SIMD, enough to hide a row's dependent
+// steps behind the other waves' instructions.
+constexpr uint32_t kTbWaves = 4096;
+
+struct WaveCaps {
+  uint32_t arena, rows, ops;     // a wave's bytes of the arena, rows, ops
+  uint32_t max_rows, max_query;  // rows the side may have, longest query
+  uint32_t stride;               // bytes per wave
+};
+
+// Records the operations of WaveDp's rows in the reference's layout.  A row's
+// cells past its new band end are overwritten by the following rows or never
+// read but as unwritten, so a row stores the columns [start, new end) only
+// and every byte has one writer.
+struct ArenaOps {
+  uint8_t *arena;
+  int2 *rows;  // (base, off)
+  uint32_t max_rows, extra;
+  int gap_init, gap_ext;
+  uint32_t used = 0;
+  int start = 0;  // the row's first column in the window
+  bool full = false;
+  int op[4];
+
+  static __device__ __forceinline__ uint32_t Need(uint32_t length) { return length + length / 3; }
+
+  __device__ __forceinline__ bool Row(const WaveDpBand &B) {
+    const uint32_t as = (uint32_t)(B.base + B.start);
+    const uint32_t length = gap_ext > 0 ? (uint32_t)(B.end - B.start) + extra : extra - as;
+    if ((uint64_t)used + Need(length) >= kTracebackArena || (uint32_t)B.row >= max_rows) {
+      full = true;
+      return false;
+    }
+    if (__lane_id() == 0) rows[B.row] = make_int2((int)used + 1, (int)as);
+    start = B.start;
+    return true;
+  }
+
+  template <class Dp, int C>
+  __device__ __forceinline__ void Cells(const Dp &dp, const WaveDpParams &P, const WaveDpBand &B,
+                                        const uint64_t (&live)[C], const int (&s)[C],
+                                        const int (&diag)[C], const int (&sp)[C],
+                                        const int (&gap)[C]) {
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const int a = Dp::Offset(j), opened = s[j] - gap_init;
+      int x = diag[j] < dp.e[j] ? kGap0 : kSub;
+      x = sp[j] < gap[j] ? kGap1 : x;
+      x += dp.e[j] - gap_ext >= opened ? kExt0 : 0;
+      x += gap[j] - gap_ext >= opened ? kExt1 : 0;
+      // the band's first column and those a row's gap appends
+      const bool fixed = a == B.start || a >= B.end;
+      x = fixed ? kGap0 + kExt0 : x;
+      const bool kept = __builtin_amdgcn_inverse_ballot_w64(live[j]) || a == B.start;
+      op[j] = kept ? x : kUnwritten;
+    }
+  }
+
+  template <class Dp>
+  __device__ __forceinline__ void End(const Dp &, const WaveDpBand &B, bool any) {
+    constexpr int C = Dp::W / kWave;
+    // nothing kept: the side's last row; only its first column can be read
+    const int columns = any ? B.end - start : 1;
+    uint8_t *row = arena + used + 1;
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const int k = Dp::Offset(j) - start;
+      if (k >= 0 && k < columns) row[k] = (uint8_t)op[j];
+    }
+    used += (uint32_t)columns;
+  }
+};
+
+// One side: q0 / d0 the positions of its first residues, s0len the distance
+// to the query's end.
+template <bool kReverse>
+__device__ void WaveSide(const WaveDpParams &P, const int8_t *sm, uint32_t q0, uint32_t s0len,
+                         uint32_t d0, uint8_t *mine, const WaveCaps &caps, TracebackHalf *out) {
+  const int lane = (int)__lane_id();
+  ArenaOps ops;
+  ops.arena = mine;
+  ops.rows = reinterpret_cast<int2 *>(mine + caps.arena);
+  ops.max_rows = caps.max_rows;
+  ops.gap_init = P.gap_init;
+  ops.gap_ext = P.gap_ext;
+  ops.extra = P.gap_ext > 0 ? (uint32_t)(P.cutoff / P.gap_ext + 3) : s0len + 3;
+  uint8_t *script = mine + caps.arena + caps.rows;
+  TracebackHalf h = {};
+  // a window of 64 columns serves a query side that ends inside it, wider
+  // ones a band that moves along its query side
+  WaveDpBand B;
+  WaveDp<kReverse, 1> x;
+  int r = x.Begin(P, B, q0, d0);
+  const bool begun = r != kWaveDpDone;
+  if (begun && ArenaOps::Need(ops.extra) >= kTracebackArena) {
+    h.flags = kTracebackOverflow;
+    if (lane == 0) *out = h;
+    return;
+  }
+  if (begun) {
+    if (r == 0 && x.EndsInside(B)) {
+      r = x.Rows(P, sm, B, ops);
+    } else {
+      WaveDp<kReverse, 2> y;
+      r = y.Begin(P, B, q0, d0);
+      if (r == 0) r = y.Rows(P, sm, B, ops);
+      if (r == kWaveDpWiden || (r == kWaveDpLost && B.row == 0 && !ops.full)) {
+        WaveDp<kReverse, 4> z;
+        if (r == kWaveDpWiden) {
+          z.Widen(P, B, y);
+          r = 0;
+        } else {
+          r = z.Begin(P, B, q0, d0);
+        }
+        if (r == 0) r = z.Rows(P, sm, B, ops);
+      }
+    }
+  }
+  if (r != kWaveDpDone) {
+    h.flags = ops.full ? kTracebackOverflow : kNeedsLane;
+    if (lane == 0) *out = h;
+    return;
+  }
+  if (lane == 0) ops.arena[0] = kSub;
+  // the wave's stores are read by its other lanes from here on
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  // the path from the best cell back: while the state (a substitution run, a
+  // vertical or a horizontal gap) lasts, lane l looks l cells ahead
+  const int best_row = B.best_row, best_col = B.best_col;
+  int row = best_row, col = best_col, state = kSub;
+  uint32_t nops = 0;
+  while (row >= 0 && col >= 1) {
+    const int lr = row - (state != kGap1 ? lane : 0), lc = col - (state != kGap0 ? lane : 0);
+    const bool on = lr >= 0 && lc >= 1;
+    int byte = 0;
+    bool stale = false;
+    if (on) {
+      const int2 at = ops.rows[lr];
+      const int idx = at.x + lc - at.y;
+      stale = idx < 0 || idx > (int)ops.used;
+      if (!stale) {
+        byte = ops.arena[idx];
+        stale = byte == kUnwritten;
+        byte = stale ? 0 : byte;
+      }
+    }
+    const bool go = on && (state == kSub ? (byte & 3) == 0
+                                         : (byte & (state == kGap0 ? kExt0 : kExt1)) != 0);
+    const uint64_t stops = __ballot(!go), inside = __ballot(on);
+    const int f = stops ? __ffsll((unsigned long long)stops) - 1 : kWave;
+    const bool turns = f < kWave && ((inside >> f) & 1ull) != 0;
+    // the cells that the path visits
+    const uint64_t seen = f >= kWave - 1 ? ~0ull : (2ull << f) - 1ull;
+    if (__ballot(stale) & seen) h.flags |= kTracebackStale;
+    const int next = turns ? __builtin_amdgcn_readlane(byte, f) & 3 : 0;
+    auto edit = [](int op) { return op == kGap0 ? kEditGap0 : op == kGap1 ? kEditGap1 : kEditSub; };
+    if (lane < f || (lane == f && turns)) script[nops + lane] = edit(lane < f ? state : next);
+    row -= state != kGap1 ? f : 0;
+    col -= state != kGap0 ? f : 0;
+    nops += (uint32_t)f;
+    if (turns) {
+      ++nops;
+      row -= next != kGap1 ? 1 : 0;
+      col -= next != kGap0 ? 1 : 0;
+      state = next;
+    }
+  }
+  const int tail = row >= 0 ? row + 1 : col >= 1 ? col : 0;
+  for (int k = lane; k < tail; k += kWave) script[nops + k] = row >= 0 ? kEditGap0 : kEditGap1;
+  nops += (uint32_t)tail;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  // The joined script holds both generated sequences reversed, the reverse
+  // side's first: each side's counts stand alone, since a side consumes
+  // exactly its stretch of both sequences and the reverse side's last op (its
+  // first generated one, at the best cell) is never a gap.
+  const int inc = kReverse ? -1 : 1;
+  h.score = B.best;
+  h.q = q0 + (uint32_t)((best_col - 1) * inc);
+  h.d = d0 + (uint32_t)(best_row * inc);
+  uint32_t q = kReverse ? h.q : q0, d = kReverse ? h.d : d0;
+  uint64_t last0 = 0, last1 = 0;  // whether the pass before ended in a gap
+  const uint64_t below = (1ull << lane) - 1ull;
+  for (uint32_t k = 0; k < nops; k += kWave) {
+    const bool on = k + (uint32_t)lane < nops;
+    const int e = on ? script[nops - 1 - k - (uint32_t)lane] : -1;
+    const uint64_t subs = __ballot(e == kEditSub), gap0 = __ballot(e == kEditGap0),
+                   gap1 = __ballot(e == kEditGap1);
+    bool differs = false;
+    if (e == kEditSub)
+      differs = CodeAt(P.queries, q + (uint32_t)__popcll((subs | gap1) & below)) !=
+                CodeAt(P.database, d + (uint32_t)__popcll((subs | gap0) & below));
+    h.mismatches += (uint32_t)__popcll(__ballot(differs));
+    const uint32_t opens = (uint32_t)(__popcll(gap0 & ~(gap0 << 1 | last0)) +
+                                      __popcll(gap1 & ~(gap1 << 1 | last1)));
+    h.gap_openings += opens;
+    h.gap_extensions += (uint32_t)(__popcll(gap0) + __popcll(gap1)) - opens;
+    last0 = gap0 >> 63;
+    last1 = gap1 >> 63;
+    q += (uint32_t)__popcll(subs | gap1);
+    d += (uint32_t)__popcll(subs | gap0);
+  }
+  h.length = nops;
+  if (lane == 0) *out = h;
+}
+
+// Sides of the jobs, one wave each: blocks of even index the reverse sides
+// (from hit - 1), of odd index the forward sides.  A wave takes `batch` jobs
+// at a time, its first without asking, the others from heads[direction]
+// (zero at the launch).
+//
+// Bound: the issue of a row's instructions (with the operations about 120,
+// against 90 without), then the path's dependent loads, a table entry and an
+// op per run of equal operations.  A call with its copies, against a lane per
+// result that walks the cells one by one with its op rows strided over the
+// chip's memory: 50,021 results of reads 5.9 -> 1.7 ms, 3,001 of proteins of
+// 100-500 residues 26 -> 1.0 ms.
+__global__ void __launch_bounds__(kTbWaveBlock)
+    TracebackWaveKernel(WaveDpParams P, const TracebackJob *jobs, uint32_t n, uint32_t batch,
+                        uint32_t *heads, const int *matrix, uint32_t nl, uint8_t *scratch,
+                        WaveCaps caps, TracebackHalf *halves) {
+  __shared__ int8_t sm[kTableDim * kScoreStride];
+  StageWaveDpScores(sm, matrix, nl);
+  __syncthreads();
+  const uint32_t side = blockIdx.x & 1u, per = kTbWaveBlock / kWave;
+  const uint32_t in_block = Uniform(threadIdx.x / kWave);
+  const uint32_t wave = (blockIdx.x >> 1) * per + in_block;
+  const uint32_t waves = (gridDim.x >> 1) * per;
+  uint8_t *mine = scratch + (size_t)(blockIdx.x * per + in_block) * caps.stride;
+  for (uint32_t first = wave * batch; first < n;) {
+    const uint32_t stop = first + batch < n ? first + batch : n;
+    for (uint32_t j = first; j < stop; ++j) {
+      const uint32_t offset = Uniform(jobs[j].query_offset), length = Uniform(jobs[j].query_length);
+      const uint32_t hit_q = Uniform(jobs[j].hit_q), hit_d = Uniform(jobs[j].hit_d);
+      TracebackHalf *out = halves + 2 * (size_t)j + side;
+      // the buffers hold any side between the query's two delimiters
+      const bool framed = hit_q >= 1 && hit_q < length && length <= caps.max_query &&
+                          CodeAt(P.queries, offset) == kDelimiter &&
+                          CodeAt(P.queries, (int64_t)offset + length - 1) == kDelimiter;
+      if (!Uniform(framed ? 1 : 0)) {
+        if (__lane_id() == 0) {
+          TracebackHalf h = {};
+          h.flags = kNeedsLane;
+          *out = h;
+        }
+      } else if (side == 0) {
+        WaveSide<true>(P, sm, offset + hit_q - 1, hit_q - 1, hit_d - 1, mine, caps, out);
+      } else {
+        WaveSide<false>(P, sm, offset + hit_q, length - hit_q, hit_d, mine, caps, out);
+      }
+    }
+    if ((uint64_t)waves * batch >= n) break;  // no jobs past the first ones
+    uint32_t b = 0;
+    if (__lane_id() == 0) b = atomicAdd(&heads[side], batch);
+    first = waves * batch + Uniform(b);
+  }
+}
+
+// Both sides' halves as results; jobs that a wave could not serve are listed.
+__global__ void __launch_bounds__(256)
+    TracebackJoinKernel(const TracebackJob *jobs, uint32_t n, const TracebackHalf *halves,
+                        TracebackOut *outs, uint32_t *count, uint32_t *list) {
+  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= n) return;
+  const TracebackHalf rev = halves[2 * (size_t)j], fwd = halves[2 * (size_t)j + 1];
+  if ((rev.flags | fwd.flags) & kNeedsLane) {
+    list[atomicAdd(count, 1u)] = j;
+    return;
+  }
+  TracebackOut o = {};
+  o.flags = rev.flags | (rev.flags & kTracebackOverflow ? 0u : fwd.flags);
+  if (!(o.flags & kTracebackOverflow)) {
+    const uint32_t offset = jobs[j].query_offset;
+    o.score = rev.score + fwd.score;
+    o.start_q = rev.q - offset;
+    o.start_d = rev.d;
+    o.end_q = fwd.q - offset;
+    o.end_d = fwd.d;
+    o.length = rev.length + fwd.length;
+    o.mismatches = rev.mismatches + fwd.mismatches;
+    o.gap_openings = rev.gap_openings + fwd.gap_openings;
+    o.gap_extensions = rev.gap_extensions + fwd.gap_extensions;
+  }
+  outs[j] = o;
+}
+
+__global__ void ClearKernel(uint32_t *p, uint32_t n) {
+  if (threadIdx.x < n) p[threadIdx.x] = 0;
+}
+
+size_t Align256(size_t b) { return (b + 255) / 256 * 256; }
+
+// A lane's scratch capacities.
+LaneCaps TracebackCaps(uint32_t max_query_length, uint32_t max_subject_length) {
   LaneCaps c;
   c.dp = max_query_length + 4;
   c.rows = max_subject_length + 4;
-  c.arena = arena;
+  c.arena = kTracebackArena;
   c.ops = 2 * (max_query_length + max_subject_length) + 16;
-  size_t b = (size_t)(c.dp + c.rows) * sizeof(int2) + c.arena + c.ops;
-  c.bytes_per_lane = (b + 255) / 256 * 256;
+  c.bytes_per_lane = Align256((size_t)(c.dp + c.rows) * sizeof(int2) + c.arena + c.ops);
   return c;
 }
 
-hipError_t TracebackLaunch(const uint64_t *pq, const uint64_t *pd, const TracebackJob *jobs,
-                           uint32_t n, const int *matrix, uint32_t nl, int gap_open,
-                           int gap_ext, int cutoff, uint8_t *scratch, const LaneCaps &caps,
-                           uint32_t lanes, TracebackOut *outs, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  const uint32_t blocks = (lanes + kTbThreads - 1) / kTbThreads;
-  const bool short_cells = cutoff <= 8192 && gap_ext >= 0 && gap_open + gap_ext <= 1024;
+// A wave's: an arena that holds the rows a side can have, up to the limit.
+WaveCaps TracebackWaveCaps(uint32_t max_query_length, uint32_t max_subject_length) {
+  WaveCaps c;
+  const uint64_t rows = (uint64_t)max_subject_length + 4, cols = (uint64_t)max_query_length + 4;
+  c.max_rows = (uint32_t)rows;
+  c.max_query = max_query_length;
+  c.arena = (uint32_t)Align256(std::min<uint64_t>(kTracebackArena, rows * cols + 16));
+  c.rows = (uint32_t)(rows * sizeof(int2));
+  c.ops = (uint32_t)(rows + cols + 16);
+  c.stride = (uint32_t)Align256((size_t)c.arena + c.rows + c.ops);
+  return c;
+}
+
+}  // namespace
+
+TracebackRunner::~TracebackRunner() {
+  if (ws_) (void)gz::Free(ws_);
+  if (lane_ws_) (void)gz::Free(lane_ws_);
+  for (hipEvent_t e : ev_)
+    if (e) (void)hipEventDestroy(e);
+}
+
+hipError_t TracebackRunner::Reserve(void **p, size_t *cap, size_t bytes) {
+  if (*cap >= bytes) return hipSuccess;
+  if (*p) (void)gz::Free(*p);
+  *p = nullptr;
+  *cap = 0;
+  const hipError_t e = gz::Malloc(p, bytes);
+  if (e == hipSuccess) *cap = bytes;
+  return e;
+}
+
+hipError_t TracebackRunner::Lanes(const TracebackInputs &in, const TracebackJob *d_jobs,
+                                  uint32_t n, const uint32_t *d_list, TracebackOut *d_outs,
+                                  hipStream_t s) {
+  const LaneCaps caps = TracebackCaps(in.max_query_length, in.max_subject_length);
+  // lanes resident at once (up to seven 64-lane blocks per CU), bounded by a
+  // 12 GB scratch budget
+  const size_t budget = (size_t)12 << 30;
+  size_t lanes = std::min<size_t>(((size_t)n + 63) / 64 * 64, (size_t)7 * 64 * 256);
+  lanes = std::max<size_t>(64, std::min(lanes, budget / caps.bytes_per_lane / 64 * 64));
+  hipError_t e = Reserve(&lane_ws_, &lane_cap_, lanes * caps.bytes_per_lane);
+  if (e != hipSuccess) return e;
+  const uint32_t blocks = (uint32_t)(lanes / kTbThreads);
+  const bool short_cells =
+      in.cutoff <= 8192 && in.gap_ext >= 0 && in.gap_open + in.gap_ext <= 1024;
   if (short_cells)
-    hipLaunchKernelGGL(TracebackKernel<true>, dim3(blocks), dim3(kTbThreads), 0, s, pq, pd, jobs,
-                       n, matrix, nl, gap_open, gap_ext, cutoff, scratch, caps, outs);
+    hipLaunchKernelGGL(TracebackKernel<true>, dim3(blocks), dim3(kTbThreads), 0, s, in.queries,
+                       in.database, d_jobs, n, d_list, in.matrix, in.nl, in.gap_open, in.gap_ext,
+                       in.cutoff, (uint8_t *)lane_ws_, caps, d_outs);
   else
-    hipLaunchKernelGGL(TracebackKernel<false>, dim3(blocks), dim3(kTbThreads), 0, s, pq, pd,
-                       jobs, n, matrix, nl, gap_open, gap_ext, cutoff, scratch, caps, outs);
+    hipLaunchKernelGGL(TracebackKernel<false>, dim3(blocks), dim3(kTbThreads), 0, s, in.queries,
+                       in.database, d_jobs, n, d_list, in.matrix, in.nl, in.gap_open, in.gap_ext,
+                       in.cutoff, (uint8_t *)lane_ws_, caps, d_outs);
   return hipGetLastError();
+}
+
+hipError_t TracebackRunner::Run(const TracebackInputs &in, const TracebackJob *jobs, uint32_t n,
+                                TracebackOut *outs, hipStream_t s, float *kernel_ms) {
+  if (n == 0) return hipSuccess;
+  for (hipEvent_t &x : ev_)
+    if (!x) {
+      const hipError_t c = hipEventCreate(&x);
+      if (c != hipSuccess) return c;
+    }
+  // the wave form's rows of the longest subject must fit 32-bit offsets
+  const bool waves = WaveDpServes(in.cutoff, in.gap_open, in.gap_ext) &&
+                     in.max_subject_length < (1u << 27) && in.max_query_length < (1u << 27);
+  const uint32_t per = kTbWaveBlock / kWave;
+  WaveCaps wc = {};
+  uint32_t side_blocks = 0, batch = 1;
+  if (waves) {
+    wc = TracebackWaveCaps(in.max_query_length, in.max_subject_length);
+    // waves of a side: as many as jobs up to half the resident ones, within
+    // a 4 GB scratch budget
+    uint64_t side_waves = std::min<uint64_t>(n, kTbWaves / 2);
+    side_waves = std::min<uint64_t>(side_waves, ((uint64_t)4 << 30) / 2 / wc.stride);
+    side_blocks = (uint32_t)std::max<uint64_t>(1, (side_waves + per - 1) / per);
+    const uint64_t b = n / ((uint64_t)side_blocks * per * 8) + 1;
+    batch = (uint32_t)std::min<uint64_t>(b, 4);
+  }
+  const size_t a_jobs = Align256(n * sizeof(TracebackJob));
+  const size_t a_outs = Align256(n * sizeof(TracebackOut));
+  const size_t a_half = waves ? Align256(2 * (size_t)n * sizeof(TracebackHalf)) : 0;
+  const size_t a_list = waves ? Align256((size_t)n * 4) : 0;
+  const size_t a_wave = (size_t)side_blocks * 2 * per * wc.stride;
+  hipError_t e = Reserve(&ws_, &cap_, a_jobs + a_outs + 256 + a_half + a_list + a_wave);
+  if (e != hipSuccess) return e;
+  char *w = (char *)ws_;
+  TracebackJob *d_jobs = (TracebackJob *)w;
+  TracebackOut *d_outs = (TracebackOut *)(w + a_jobs);
+  uint32_t *d_counters = (uint32_t *)(w + a_jobs + a_outs);  // heads, listed jobs
+  TracebackHalf *d_halves = (TracebackHalf *)(w + a_jobs + a_outs + 256);
+  uint32_t *d_list = (uint32_t *)(w + a_jobs + a_outs + 256 + a_half);
+  uint8_t *scratch = (uint8_t *)(w + a_jobs + a_outs + 256 + a_half + a_list);
+  e = hipMemcpyAsync(d_jobs, jobs, n * sizeof(TracebackJob), hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) e = hipEventRecord(ev_[0], s);
+  if (e != hipSuccess) return e;
+  uint32_t listed = 0;
+  if (waves) {
+    const WaveDpParams P = {in.queries, in.database, kDelimiter, in.gap_open + in.gap_ext,
+                            in.gap_ext, in.cutoff,
+                            in.gap_ext > 0 ? std::max(in.cutoff - in.gap_open - in.gap_ext, 0) /
+                                                 in.gap_ext + 2
+                                           : kWaveDpMargin};
+    hipLaunchKernelGGL(ClearKernel, dim3(1), dim3(64), 0, s, d_counters, 3u);
+    hipLaunchKernelGGL(TracebackWaveKernel, dim3(2 * side_blocks), dim3(kTbWaveBlock), 0, s, P,
+                       d_jobs, n, batch, d_counters, in.matrix, in.nl, scratch, wc, d_halves);
+    hipLaunchKernelGGL(TracebackJoinKernel, dim3((n + 255) / 256), dim3(256), 0, s, d_jobs, n,
+                       d_halves, d_outs, d_counters + 2, d_list);
+    e = hipGetLastError();
+  } else {
+    e = Lanes(in, d_jobs, n, nullptr, d_outs, s);
+  }
+  if (e == hipSuccess) e = hipEventRecord(ev_[1], s);
+  // the copies back are queued once the kernels are done: a device-to-host
+  // copy queued behind a running kernel holds up other streams' copies
+  if (e == hipSuccess) e = hipEventSynchronize(ev_[1]);
+  if (e == hipSuccess && waves) {
+    e = hipMemcpyAsync(&listed, d_counters + 2, 4, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e == hipSuccess && listed > 0) {
+      // bands past 256 columns and jobs whose frame is not as described
+      e = Lanes(in, d_jobs, listed, d_list, d_outs, s);
+      if (e == hipSuccess) e = hipEventRecord(ev_[1], s);
+      if (e == hipSuccess) e = hipEventSynchronize(ev_[1]);
+    }
+  }
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(outs, d_outs, n * sizeof(TracebackOut), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e == hipSuccess && kernel_ms) e = hipEventElapsedTime(kernel_ms, ev_[0], ev_[1]);
+  return e;
 }
 
 }  // namespace gz

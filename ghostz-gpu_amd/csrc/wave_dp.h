@@ -83,7 +83,15 @@ struct WaveDpParams {
   int gap_init;  // gap open + extension
   int gap_ext;
   int cutoff;
+  // columns kept free behind the band while its query side goes on past the
+  // window: a row's gap fills at most (cutoff - gap_init) / gap_ext + 1 (a
+  // row that fills more is noticed at the next one)
+  int margin;
 };
+
+// Margin of the score-only form: what the presearch's parameters (26, 12, 1)
+// need; wider gaps are rare and end in the global ring.
+constexpr int kWaveDpMargin = 16;
 
 // The value of a wave-uniform expression as a scalar.
 __device__ __forceinline__ int Uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -121,10 +129,6 @@ struct WaveDpBand {
 template <bool kReverse, int C>
 struct WaveDp {
   static constexpr int W = kWave * C;
-  // columns kept free behind the band: a row's gap fills at most
-  // (cutoff - gap_init) / gap_ext + 1, 15 at the presearch's parameters (a
-  // row that fills more is noticed at the next one)
-  static constexpr int kMargin = 16;
   // A read of C <= 12 codes touches two packed words, 24 codes from the
   // first's word on; new columns are read at most this far past a residue,
   // which keeps the words inside the delimiter padding.
@@ -138,6 +142,12 @@ struct WaveDp {
 
   static __device__ __forceinline__ int Lane() { return (int)__lane_id(); }
   static __device__ __forceinline__ int Offset(int j) { return Lane() * C + j; }
+
+  // Whether the query side ends inside the window (with room for the shifts
+  // by `start`, which then is at most W - C - 2).
+  static __device__ __forceinline__ bool EndsInside(const WaveDpBand &B) {
+    return B.last_col - B.base < W - C;
+  }
 
   // The codes of the lane's columns (column c >= 1 is the query code at
   // qpos + (c - 1) inc); every one must lie within kReach of a residue.
@@ -306,8 +316,10 @@ struct WaveDp {
     int score[C];
     LoadScores(sm, score, B.d);
     for (;;) {
-      // what a row rarely needs: room behind the band
-      while (B.end + kMargin > W) {
+      // what a row rarely needs: room behind the band, unless the query side
+      // ends inside the window (the band then ends with it)
+      int room = W - P.margin;
+      while (!EndsInside(B) && B.end > room) {
         // a live column at the window's end: the gap may go on outside
         if (B.end > W) return kWaveDpLost;
         int lanes = B.start / C;
@@ -316,6 +328,7 @@ struct WaveDp {
         Rebase(P, B, lanes);
         LoadScores(sm, score, B.d);
       }
+      if (EndsInside(B)) room = W;
       // and a cleared diagonal
       if (B.bare) {
 #pragma unroll
@@ -330,7 +343,7 @@ struct WaveDp {
         const uint32_t dn = NextCode(P, B);
         int next[C];
         LoadScores(sm, next, dn);
-        int sp[C], s[C], diag[C];
+        int sp[C], s[C], diag[C], gap[C];
         {
           int prev = WaveShiftUp1(h[C - 1], kInitScore);
           int total = 0;  // the best gap source, as the gap into the lane's following column
@@ -347,6 +360,7 @@ struct WaveDp {
           int g = WaveShiftUp1(WaveMaxScan(total + key_add), kNoScore) - key_sub;
 #pragma unroll
           for (int j = 0; j < C; ++j) {
+            gap[j] = g;
             // max(sp, g), or at most sp (a wall) past the last residue
             asm("v_med3_i32 %0, %1, %2, %3" : "=v"(s[j]) : "v"(sp[j]), "v"(g), "v"(limit[j]));
             if (j + 1 < C) {
@@ -418,7 +432,7 @@ struct WaveDp {
             last = past[j] && hi > last ? hi : last;
           }
         }
-        ops.Cells(*this, P, B, live, s, diag, sp);
+        ops.Cells(*this, P, B, live, s, diag, sp, gap);
         // the old first column leaves the band when the band's start moves
         // (nothing kept: the row is the last one)
         const bool moved = first - 1 != B.start;
@@ -447,31 +461,32 @@ struct WaveDp {
         for (int j = 0; j < C; ++j) score[j] = next[j];
         // the loop's exits: nothing kept, the database's delimiter, no room,
         // or a diagonal to clear
-        stop = ((int)(dn ^ P.delim) - 1) | (W - kMargin - B.end) | B.bare;
+        stop = ((int)(dn ^ P.delim) - 1) | (room - B.end) | B.bare;
         if (any == 0) stop = -1;
-        ops.End(B);
+        ops.End(*this, B, any != 0);
       } while (stop >= 0);
       if (any == 0 || B.d == P.delim) return kWaveDpDone;
     }
   }
 
-  // Takes over the row of a window of one column per lane, lane l's columns
-  // becoming those of lanes l C .. l C + C - 1.
+  // Takes over the row of a window of C / 2 columns per lane: column c of the
+  // window moves from lane c / (C / 2) to lane c / C.
   __device__ __forceinline__ void Widen(const WaveDpParams &P, WaveDpBand &B,
-                                        const WaveDp<kReverse, 1> &x) {
+                                        const WaveDp<kReverse, C / 2> &x) {
+    constexpr int H = C / 2;
 #pragma unroll
     for (int j = 0; j < C; ++j) {
-      const int from = Offset(j);
+      const int from = 2 * Lane() + j / H;
       const bool inside = from < kWave;
       const int at = 4 * (inside ? from : 0);
-      const int vh = __builtin_amdgcn_ds_bpermute(at, x.h[0]);
-      const int ve = __builtin_amdgcn_ds_bpermute(at, x.e[0]);
-      const int vc = __builtin_amdgcn_ds_bpermute(at, x.code[0]);
+      const int vh = __builtin_amdgcn_ds_bpermute(at, x.h[j % H]);
+      const int ve = __builtin_amdgcn_ds_bpermute(at, x.e[j % H]);
+      const int vc = __builtin_amdgcn_ds_bpermute(at, x.code[j % H]);
       h[j] = inside ? vh : kInitScore;
       e[j] = inside ? ve : kInitScore;
       code[j] = inside ? vc : kWallCode;
     }
-    ReadWindow(P, B, kWave);
+    ReadWindow(P, B, kWave * H);
     Limits(B);
   }
 };
@@ -482,8 +497,9 @@ struct NoOps {
   template <class Dp, int C>
   __device__ __forceinline__ void Cells(const Dp &, const WaveDpParams &, const WaveDpBand &,
                                         const uint64_t (&)[C], const int (&)[C],
-                                        const int (&)[C], const int (&)[C]) {}
-  __device__ __forceinline__ void End(const WaveDpBand &) {}
+                                        const int (&)[C], const int (&)[C], const int (&)[C]) {}
+  template <class Dp>
+  __device__ __forceinline__ void End(const Dp &, const WaveDpBand &, bool) {}
 };
 
 constexpr int kWaveDpBlock = 256;

@@ -1,0 +1,146 @@
+"""The result build with one wave per side (traceback.hip) against the host
+result build and the CPU oracle.  All fields are whole numbers and are
+compared exactly; a result that reads a byte an earlier extension left must be
+flagged as the host flags it."""
+import numpy as np
+import pytest
+
+import gz_native as gz
+import oracle_py
+from helpers import DELIM, concat, mutate, random_protein
+
+pytestmark = pytest.mark.gpu
+STALE, OVERFLOW = 1, 2
+
+
+def jobs_of(rng, lengths, identity, indel, at=None):
+    """Related pairs, one job each: the seed at `at` (a share of the shorter
+    sequence; None: anywhere) on a shared diagonal."""
+    qs, ds = [], []
+    for n in lengths:
+        a = random_protein(rng, int(n), 0.02)
+        b = mutate(rng, a, rng.uniform(*identity), indel)
+        qs.append(a)
+        ds.append(b if len(b) > 1 else random_protein(rng, 3))
+    q, qo = concat(qs)
+    d, do = concat(ds)
+    jobs = np.zeros((len(qs), 4), np.uint32)
+    for i, (a, b) in enumerate(zip(qs, ds)):
+        m = min(len(a), len(b))
+        k = int(rng.integers(0, m)) if at is None else min(m - 1, int(at * m))
+        jobs[i] = qo[i] - 1, len(a) + 2, k + 1, do[i] + k
+    return q, d, jobs, int(np.diff(do.astype(np.int64)).max())
+
+
+def build(q, d, jobs, max_subject, cutoff, gap_open=11, gap_ext=1, max_query=None):
+    m, nl = gz.blosum62()
+    _, pq = gz.pack_on_device(q)
+    _, pd = gz.pack_on_device(d)
+    dm = gz.DeviceBuffer.from_array(m)
+    jobs = np.ascontiguousarray(jobs)
+    out = np.zeros((len(jobs), 10), np.uint32)
+    gz.check(gz.lib().gz_build_results(
+        pq.ptr, pd.ptr, gz.ptr(jobs), len(jobs),
+        int(jobs[:, 1].max()) if max_query is None else max_query, max_subject, dm.ptr, nl,
+        gap_open, gap_ext, cutoff, gz.ptr(out), None))
+    return out
+
+
+def on_host(q, d, job, cutoff):
+    lead, qlen, hq, hd = (int(x) for x in job)
+    qs = np.ascontiguousarray(q[lead:lead + qlen])
+    out = np.zeros(10, np.uint32)
+    gz.check(gz.lib().gz_build_result_host(gz.ptr(qs), qlen, gz.ptr(d), hq, hd, cutoff,
+                                           gz.ptr(out)))
+    return out
+
+
+def by_oracle(q, d, job, cutoff, gap_open, gap_ext):
+    """The joined script's counts: the reverse side's operations in origin
+    order first, then the forward side's."""
+    m, nl = gz.blosum62()
+    lead, qlen, hq, hd = (int(x) for x in job)
+    s0, a0, b0, rev, _ = oracle_py.gapped_one_side(
+        "oracle", q, lead + hq - 1, hq - 1, d, hd - 1, DELIM, True, m, nl, gap_open, gap_ext,
+        cutoff, traceback=True)
+    s1, a1, b1, fwd, _ = oracle_py.gapped_one_side(
+        "oracle", q, lead + hq, qlen - hq, d, hd, DELIM, False, m, nl, gap_open, gap_ext, cutoff,
+        traceback=True)
+    return s0 + s1, hq - 1 + a0, hd - 1 + b0, hq + a1, hd + b1, len(rev) + len(fwd)
+
+
+# sides that end inside the 64-column window, at its edge and past it; bands
+# that stay in the 128- and 256-column windows and that outgrow them (the last
+# go to the lanes)
+@pytest.mark.parametrize("cutoff,lengths", [
+    (52, (1, 2, 3, 12, 13, 24, 25, 49, 61, 62, 63, 64, 65, 66, 67)),
+    (52, (125, 126, 127, 128, 129, 130, 400)), (26, (30, 64, 300)), (8, (30, 90)), (0, (20,)),
+    (75, (64, 128, 300)), (120, (62, 64, 126, 128, 254, 256, 500, 900))])
+@pytest.mark.parametrize("at", [None, 0.0, 1.0])
+def test_waves_vs_host(cutoff, lengths, at):
+    rng = np.random.default_rng(cutoff + len(lengths))
+    print("traceback waves: cutoff", cutoff, "lengths", lengths, "seed", at, flush=True)
+    q, d, jobs, most = jobs_of(rng, np.repeat(lengths, 16), (0.3, 1.0), 0.05, at)
+    out = build(q, d, jobs, most, cutoff)
+    stale = 0
+    for k, job in enumerate(jobs):
+        if out[k, 9] & OVERFLOW:  # 500 rows of bands past 130 columns fill the arena
+            assert job[1] * 230 > 1 << 16
+            continue
+        host = on_host(q, d, job, cutoff)
+        assert out[k, 9] == host[9], (k, job, out[k], host)
+        stale += int(host[9])
+        if not host[9]:
+            assert np.array_equal(out[k], host), (k, job, out[k], host)
+    print("  stale", stale, flush=True)
+
+
+@pytest.mark.parametrize("cutoff,gap_open,gap_ext", [
+    (52, 11, 1), (60, 0, 3), (35, 8, 0), (52, 5, 2), (120, 30, 1), (10, 11, 1)])
+def test_waves_vs_oracle(cutoff, gap_open, gap_ext):
+    """Other gap costs: scores, both ends and the script's length."""
+    rng = np.random.default_rng(cutoff + 3 * gap_open)
+    print("traceback waves: cutoff", cutoff, "gaps", gap_open, gap_ext, flush=True)
+    q, d, jobs, most = jobs_of(rng, np.repeat((40, 63, 64, 130, 260), 20), (0.4, 1.0), 0.04)
+    out = build(q, d, jobs, most, cutoff, gap_open, gap_ext)
+    served = 0
+    for k, job in enumerate(jobs):
+        if out[k, 9]:
+            continue
+        served += 1
+        got = tuple(int(x) for x in out[k, :6].astype(np.int64))
+        want = by_oracle(q, d, job, cutoff, gap_open, gap_ext)
+        assert got == want, (k, job, got, want)
+    assert served > len(jobs) // 2
+
+
+def test_more_jobs_than_waves():
+    """Jobs past the resident waves' first ones, and their order in the call."""
+    rng = np.random.default_rng(5)
+    q, d, jobs, most = jobs_of(rng, rng.integers(2, 150, 700), (0.3, 1.0), 0.05)
+    pick = rng.integers(0, len(jobs), 30011)
+    print("traceback waves:", len(pick), "jobs", flush=True)
+    one, many = build(q, d, jobs, most, 52), build(q, d, jobs[pick], most, 52)
+    assert np.array_equal(one[pick], many)
+    assert np.array_equal(one[:1], build(q, d, jobs[:1], most, 52))
+
+
+def test_bounds_of_the_call():
+    """Subjects longer than described: flagged once a side has more rows than
+    described; a longest query that is too small: sides of up to 62 residues
+    are built, longer ones flagged; a window of a query (no delimiter where
+    its frame ends) is built as before."""
+    rng = np.random.default_rng(6)
+    q, d, jobs, most = jobs_of(rng, np.repeat((30, 61, 200), 40), (0.9, 1.0), 0.0, 0.0)
+    full = build(q, d, jobs, most, 52)
+    print("traceback bounds", flush=True)
+    few = build(q, d, jobs, 40, 52)
+    long = jobs[:, 1] > 100
+    assert np.array_equal(few[:40], full[:40])
+    assert (few[long, 9] & OVERFLOW).all() and (few[long, :9] == 0).all()
+    small = build(q, d, jobs, most, 52, max_query=20)
+    assert np.array_equal(small[~long], full[~long])
+    assert (small[long, 9] & OVERFLOW).all()
+    part = jobs.copy()
+    part[:, 1] -= 3  # the frame ends before the query's delimiter
+    assert np.array_equal(build(q, d, part, most, 52), full)
