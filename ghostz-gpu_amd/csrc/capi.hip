@@ -35,6 +35,68 @@ std::recursive_mutex &gz::CaptureLock() {
   return m;
 }
 
+namespace {
+
+struct KeptBlock {
+  void *p = nullptr;
+  size_t capacity = 0;
+};
+constexpr int kPoolDevices = 64;
+std::mutex &PoolMutex() {
+  static std::mutex m;
+  return m;
+}
+KeptBlock g_kept[kPoolDevices];
+
+}  // namespace
+
+hipError_t gz::WorkspacePool::Take(size_t bytes, void **p, size_t *capacity) {
+  int dev = 0;
+  const hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (dev >= 0 && dev < kPoolDevices) {
+    std::lock_guard<std::mutex> lock(PoolMutex());
+    KeptBlock &k = g_kept[dev];
+    if (k.p && k.capacity >= bytes) {
+      *p = k.p;
+      *capacity = k.capacity;
+      k = KeptBlock();
+      return hipSuccess;
+    }
+  }
+  *capacity = bytes;
+  return gz::Malloc(p, bytes);
+}
+
+void gz::WorkspacePool::Give(void *p, size_t capacity) {
+  int dev = 0;
+  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kPoolDevices && capacity <= kMost) {
+    std::lock_guard<std::mutex> lock(PoolMutex());
+    KeptBlock &k = g_kept[dev];
+    if (capacity > k.capacity) {
+      std::swap(p, k.p);
+      k.capacity = capacity;
+    }
+  }
+  if (p) (void)gz::Free(p);
+}
+
+bool gz::WorkspacePool::Trim() {
+  bool any = false;
+  for (int dev = 0; dev < kPoolDevices; ++dev) {
+    void *p = nullptr;
+    {
+      std::lock_guard<std::mutex> lock(PoolMutex());
+      p = g_kept[dev].p;
+      g_kept[dev] = KeptBlock();
+    }
+    if (!p) continue;
+    (void)gz::Free(p);
+    any = true;
+  }
+  return any;
+}
+
 struct gz_aligner_s {
   std::vector<int> matrix;
   AlignerOptions opt;
@@ -402,7 +464,7 @@ gz_status gz_build_results(const uint64_t *pq, const uint64_t *pd, const gz_trac
   hipStream_t s = stream ? stream->s : nullptr;
   const TracebackInputs in = {pq,       pd,      max_query_length, max_subject_length, d_matrix, nl,
                               gap_open, gap_ext, cutoff};
-  TracebackRunner run;
+  TracebackRunner run(/*pooled=*/true);
   const hipError_t e = run.Run(in, reinterpret_cast<const TracebackJob *>(jobs), (uint32_t)n,
                                reinterpret_cast<TracebackOut *>(results), s, nullptr);
   GZ_HIP_CHECK(e);

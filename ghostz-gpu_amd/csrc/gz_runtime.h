@@ -19,9 +19,32 @@ namespace gz {
 // allocation or free it makes mid-run hold this lock.
 std::recursive_mutex &CaptureLock();
 
+// Device workspaces of calls that have no handle to keep one.  A call takes a
+// block, is its only user until its kernels and copies have ended, and gives
+// it back; one block per device is kept between calls, of at most kMost
+// bytes, the largest given back (a call that finds none, or one too small,
+// allocates its own).  Mapping and unmapping a call's scratch costs far more
+// than using it: 50,021 read results (140 MB of scratch) take 11 ms with an
+// allocation per call and 1.34 ms without where other allocations of the
+// process come and go, 3,001 protein results (300 MB) 12 and 0.67 ms.
+class WorkspacePool {
+ public:
+  static constexpr size_t kMost = (size_t)512 << 20;
+  // the current device's block: at least `bytes`, its size to *capacity
+  static hipError_t Take(size_t bytes, void **p, size_t *capacity);
+  // with the device current that the block was taken on and no work on the
+  // block in flight
+  static void Give(void *p, size_t capacity);
+  // frees the kept blocks; whether there was one
+  static bool Trim();
+};
+
 template <typename T>
 inline hipError_t Malloc(T **p, size_t bytes) {
   std::lock_guard<std::recursive_mutex> g(CaptureLock());
+  const hipError_t e = hipMalloc((void **)p, bytes);
+  if (e != hipErrorOutOfMemory || !WorkspacePool::Trim()) return e;
+  (void)hipGetLastError();
   return hipMalloc((void **)p, bytes);
 }
 

@@ -28,10 +28,11 @@ struct TracebackInputs {
   int gap_open, gap_ext, cutoff;
 };
 
-// Runs jobs, one after the other call, in a workspace that it keeps.
+// Runs jobs, one after the other call, in a workspace that it keeps (pooled:
+// that it takes from the library's pool and gives back at its end).
 class TracebackRunner {
  public:
-  TracebackRunner() = default;
+  explicit TracebackRunner(bool pooled = false) : pooled_(pooled) {}
   ~TracebackRunner();
   TracebackRunner(const TracebackRunner &) = delete;
   TracebackRunner &operator=(const TracebackRunner &) = delete;
@@ -41,10 +42,13 @@ class TracebackRunner {
                  TracebackOut *outs, hipStream_t s, float *kernel_ms);
 
  private:
-  static hipError_t Reserve(void **p, size_t *cap, size_t bytes);
+  hipError_t Queue(const TracebackInputs &in, const TracebackJob *jobs, uint32_t n,
+                   TracebackOut *outs, hipStream_t s, float *kernel_ms);
+  hipError_t Reserve(size_t bytes);
   // one lane per job (d_list: the n jobs to run)
   hipError_t Lanes(const TracebackInputs &in, const TracebackJob *d_jobs, uint32_t n,
                    const uint32_t *d_list, TracebackOut *d_outs, hipStream_t s);
+  const bool pooled_;
   void *ws_ = nullptr, *lane_ws_ = nullptr;
   size_t cap_ = 0, lane_cap_ = 0;
   hipEvent_t ev_[2] = {nullptr, nullptr};

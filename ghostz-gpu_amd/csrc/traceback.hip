@@ -739,19 +739,30 @@ WaveCaps TracebackWaveCaps(uint32_t max_query_length, uint32_t max_subject_lengt
 }  // namespace
 
 TracebackRunner::~TracebackRunner() {
-  if (ws_) (void)gz::Free(ws_);
+  if (ws_ && pooled_) WorkspacePool::Give(ws_, cap_);
+  else if (ws_) (void)gz::Free(ws_);
   if (lane_ws_) (void)gz::Free(lane_ws_);
   for (hipEvent_t e : ev_)
     if (e) (void)hipEventDestroy(e);
 }
 
-hipError_t TracebackRunner::Reserve(void **p, size_t *cap, size_t bytes) {
-  if (*cap >= bytes) return hipSuccess;
-  if (*p) (void)gz::Free(*p);
-  *p = nullptr;
-  *cap = 0;
-  const hipError_t e = gz::Malloc(p, bytes);
-  if (e == hipSuccess) *cap = bytes;
+hipError_t TracebackRunner::Reserve(size_t bytes) {
+  if (cap_ >= bytes) return hipSuccess;
+  if (ws_ && pooled_) WorkspacePool::Give(ws_, cap_);
+  else if (ws_) (void)gz::Free(ws_);
+  ws_ = nullptr;
+  cap_ = 0;
+  hipError_t e;
+  if (pooled_) {
+    e = WorkspacePool::Take(bytes, &ws_, &cap_);
+  } else {
+    e = gz::Malloc(&ws_, bytes);
+    cap_ = bytes;
+  }
+  if (e != hipSuccess) {
+    ws_ = nullptr;
+    cap_ = 0;
+  }
   return e;
 }
 
@@ -764,8 +775,15 @@ hipError_t TracebackRunner::Lanes(const TracebackInputs &in, const TracebackJob 
   const size_t budget = (size_t)12 << 30;
   size_t lanes = std::min<size_t>(((size_t)n + 63) / 64 * 64, (size_t)7 * 64 * 256);
   lanes = std::max<size_t>(64, std::min(lanes, budget / caps.bytes_per_lane / 64 * 64));
-  hipError_t e = Reserve(&lane_ws_, &lane_cap_, lanes * caps.bytes_per_lane);
-  if (e != hipSuccess) return e;
+  const size_t bytes = lanes * caps.bytes_per_lane;
+  if (lane_cap_ < bytes) {
+    if (lane_ws_) (void)gz::Free(lane_ws_);
+    lane_ws_ = nullptr;
+    lane_cap_ = 0;
+    const hipError_t e = gz::Malloc(&lane_ws_, bytes);
+    if (e != hipSuccess) return e;
+    lane_cap_ = bytes;
+  }
   const uint32_t blocks = (uint32_t)(lanes / kTbThreads);
   const bool short_cells =
       in.cutoff <= 8192 && in.gap_ext >= 0 && in.gap_open + in.gap_ext <= 1024;
@@ -783,6 +801,14 @@ hipError_t TracebackRunner::Lanes(const TracebackInputs &in, const TracebackJob 
 hipError_t TracebackRunner::Run(const TracebackInputs &in, const TracebackJob *jobs, uint32_t n,
                                 TracebackOut *outs, hipStream_t s, float *kernel_ms) {
   if (n == 0) return hipSuccess;
+  const hipError_t e = Queue(in, jobs, n, outs, s, kernel_ms);
+  // after an error nothing of the call may still use the workspace
+  if (e != hipSuccess) (void)hipStreamSynchronize(s);
+  return e;
+}
+
+hipError_t TracebackRunner::Queue(const TracebackInputs &in, const TracebackJob *jobs, uint32_t n,
+                                  TracebackOut *outs, hipStream_t s, float *kernel_ms) {
   for (hipEvent_t &x : ev_)
     if (!x) {
       const hipError_t c = hipEventCreate(&x);
@@ -809,7 +835,7 @@ hipError_t TracebackRunner::Run(const TracebackInputs &in, const TracebackJob *j
   const size_t a_half = waves ? Align256(2 * (size_t)n * sizeof(TracebackHalf)) : 0;
   const size_t a_list = waves ? Align256((size_t)n * 4) : 0;
   const size_t a_wave = (size_t)side_blocks * 2 * per * wc.stride;
-  hipError_t e = Reserve(&ws_, &cap_, a_jobs + a_outs + 256 + a_half + a_list + a_wave);
+  hipError_t e = Reserve(a_jobs + a_outs + 256 + a_half + a_list + a_wave);
   if (e != hipSuccess) return e;
   char *w = (char *)ws_;
   TracebackJob *d_jobs = (TracebackJob *)w;

@@ -2,6 +2,8 @@
 result build and the CPU oracle.  All fields are whole numbers and are
 compared exactly; a result that reads a byte an earlier extension left must be
 flagged as the host flags it."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -144,3 +146,27 @@ def test_bounds_of_the_call():
     part = jobs.copy()
     part[:, 1] -= 3  # the frame ends before the query's delimiter
     assert np.array_equal(build(q, d, part, most, 52), full)
+
+
+def test_concurrent_calls():
+    """Calls of several threads at once, of different sizes: each has a
+    workspace of its own, the kept one or a new one."""
+    rng = np.random.default_rng(7)
+    sets = [jobs_of(rng, rng.integers(2, most, n), (0.3, 1.0), 0.05)
+            for n, most in ((1500, 60), (40, 400), (600, 200))]
+    want = [build(q, d, jobs, most, 52) for q, d, jobs, most in sets]
+    print("traceback: three threads", flush=True)
+    bad = []
+
+    def work(i):
+        q, d, jobs, most = sets[i]
+        for _ in range(5):
+            if not np.array_equal(build(q, d, jobs, most, 52), want[i]):
+                bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
