@@ -3,11 +3,11 @@
 //
 // Kernels are integer-only and written for gfx950 (wave64):
 //  * PackKernel           -- PackAlphabetCodeSequence on the device
-//  * DistanceKernel       -- reduced-alphabet mismatches over a window,
-//                            one pair per lane, reduced map in LDS
+//  * DistanceKernel       -- reduced-alphabet mismatches over a window, twelve
+//                            codes a step through a class table in LDS
 //  * UngappedTriggerKernel-- reverse X-drop, forward continuation while the
-//                            sum is <= trigger; one seed per lane, the score
-//                            table in LDS, codes streamed from packed words
+//                            sum is <= trigger; one seed per lane, twelve
+//                            residues a step
 //  * SeedScatter/Gather   -- SetQuerySeeds expansion via own max-scan
 //  * GappedKernel<W>      -- the CPU's row-major affine X-drop
 //                            (src/gapped_extender.cpp:306-471), one seed per
@@ -28,6 +28,7 @@
 #include "gz_device.h"
 #include "gz_runtime.h"
 #include "gz_scan.h"
+#include "ungapped.h"
 #include "wave_dp.h"
 
 namespace gz {
@@ -53,29 +54,119 @@ __global__ void PackKernel(const uint8_t *codes, size_t n, uint64_t *packed,
 // ---------------------------------------------------------------------------
 // distance (src/distance_calculator_gpu.cu:187-286 semantics)
 // ---------------------------------------------------------------------------
+// Bound: memory.  A pair reads two packed words of each sequence, at a random
+// place or one or two cache lines past the previous pair's, so the lines
+// and not the 25 bytes of a pair are what moves.  Each code is replaced by its class's first
+// code through a table of code pairs in LDS (a read per two codes), so that
+// a window's mismatches are the non-zero five-bit fields of one exclusive
+// or; kPairs pairs are in flight per lane, each with one 16-byte read per
+// sequence (two 8-byte ones cost the address units twice the time: 112 us).
+// 4,000,003 pairs of windows of ten: 145 us with a lane that streams codes one
+// by one through cursors, 93 us so, at 4.1 TB/s of fetched lines; 1,000,003
+// pairs 26 -> 16 us.
+struct DistanceTable {
+  uint16_t pair[kTableDim * kTableDim];  // [(b << 5) | a]: classes of a and b, 5 bits each
+};
+
+// Filled from registers: lanes c and c + 32 of every wave hold the first code
+// of code c's class.
+__device__ __forceinline__ void StageDistanceTable(DistanceTable &t, const uint8_t *reduced_map) {
+  const uint32_t c = threadIdx.x % kTableDim;
+  const int v = c < kNumberLetters ? reduced_map[c] : (int)(uint8_t)(100 + c);
+  uint32_t first = c;
+#pragma unroll
+  for (int f = (int)kTableDim - 1; f >= 0; --f)
+    first = __builtin_amdgcn_readlane(v, f) == v ? (uint32_t)f : first;
+  for (uint32_t i = threadIdx.x; i < kTableDim * kTableDim; i += blockDim.x)
+    t.pair[i] = (uint16_t)(first | (uint32_t)__shfl((int)first, (int)(i / kTableDim), kWave)
+                                       << kCodeBits);
+  __syncthreads();
+}
+
+// The twelve codes from a packed position on, of which `codes` are used.  A
+// window of a whole subsequence lies at most a window past a residue, so
+// both words can be read at once (the padding behind the sequences has four);
+// of a longer subsequence's windows (kLong) the second word is read only if
+// it holds a used code.
+template <bool kLong>
+struct CodeWindow {
+  uint64_t lo, hi;
+  uint32_t k;
+  __device__ __forceinline__ void Load(const uint64_t *packed, uint32_t p, uint32_t codes) {
+    const uint32_t w = p / kCodesPerWord;
+    k = p - w * kCodesPerWord;
+    if (kLong) {
+      lo = packed[w];
+      hi = packed[w + (k + codes > kCodesPerWord ? 1 : 0)];
+    } else {
+      const WordPair v = LoadWordPair(packed + w);
+      lo = v.lo;
+      hi = v.hi;
+    }
+  }
+  __device__ __forceinline__ uint64_t Get() const {
+    return Window12(lo & kCodeBitsMask, hi & kCodeBitsMask, k);
+  }
+};
+
+// Mismatches among the first `codes` (at most 12) of two windows.
+__device__ __forceinline__ int WindowMismatches(const DistanceTable &t, uint64_t a, uint64_t b,
+                                                uint32_t codes) {
+  constexpr uint32_t kLow = 0x1ef7bdefu, kHigh = 0x21084210u;
+  int count = 0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    uint32_t x = 0;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const int at = 10 * (3 * h + p);
+      x |= (uint32_t)(t.pair[(uint32_t)(a >> at) & 1023u] ^ t.pair[(uint32_t)(b >> at) & 1023u])
+           << (10 * p);
+    }
+    const uint32_t used = codes > 6u * h ? codes - 6u * h : 0;
+    if (used < 6) x &= (1u << (kCodeBits * used)) - 1u;
+    // a field's high bit: whether the field is not zero
+    count += __popc((((x & kLow) + kLow) | x) & kHigh);
+  }
+  return count;
+}
+
+template <int kPairs, bool kLong>
 __global__ void __launch_bounds__(256)
     DistanceKernel(size_t size, const uint32_t *qcenters,
                    const uint32_t *dcenters, const uint64_t *queries,
                    const uint64_t *database, const uint8_t *reduced_map,
                    uint32_t length, char *out) {
-  __shared__ uint8_t map[kTableDim];
-  if (threadIdx.x < kTableDim) {
-    map[threadIdx.x] = (threadIdx.x < kNumberLetters)
-                           ? reduced_map[threadIdx.x]
-                           : (uint8_t)(100 + threadIdx.x);
-  }
-  __syncthreads();
-  const uint32_t half = length / 2;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < size;
-       i += (size_t)gridDim.x * blockDim.x) {
-    ForwardCursor a, b;
-    a.Init(queries, qcenters[i] - half);
-    b.Init(database, dcenters[i] - half);
-    int count = 0;
-    for (uint32_t k = 0; k < length; ++k) {
-      count += (map[a.Next()] != map[b.Next()]) ? 1 : 0;
+  __shared__ DistanceTable table;
+  StageDistanceTable(table, reduced_map);
+  const uint32_t back = length / 2 - kPackPadCodes;  // modulo 2^32
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < size; i += kPairs * stride) {
+    uint32_t qp[kPairs], dp[kPairs];
+#pragma unroll
+    for (int u = 0; u < kPairs; ++u) {
+      const size_t at = i + u * stride < size ? i + u * stride : i;
+      qp[u] = __builtin_nontemporal_load(qcenters + at) - back;
+      dp[u] = __builtin_nontemporal_load(dcenters + at) - back;
     }
-    out[i] = (char)count;
+    int count[kPairs] = {};
+    uint32_t done = 0;
+    do {
+      const uint32_t codes = length - done < kCodesPerWord ? length - done : kCodesPerWord;
+      CodeWindow<kLong> a[kPairs], b[kPairs];
+#pragma unroll
+      for (int u = 0; u < kPairs; ++u) {
+        a[u].Load(queries, qp[u] + done, codes);
+        b[u].Load(database, dp[u] + done, codes);
+      }
+#pragma unroll
+      for (int u = 0; u < kPairs; ++u)
+        count[u] += WindowMismatches(table, a[u].Get(), b[u].Get(), codes);
+      done += kCodesPerWord;
+    } while (kLong && done < length);
+#pragma unroll
+    for (int u = 0; u < kPairs; ++u)
+      if (i + u * stride < size) out[i + u * stride] = (char)count[u];
   }
 }
 
@@ -110,7 +201,7 @@ __device__ __forceinline__ int UngappedSide(Cursor &q, Cursor &d,
   return best;
 }
 
-__device__ __forceinline__ int UngappedWithTrigger(
+__device__ __forceinline__ int UngappedByResidue(
     const uint64_t *queries, uint32_t qpos, const uint64_t *database,
     uint32_t dpos, const int8_t *sm, uint32_t delim, int cutoff, int trigger) {
   ReverseCursor rq, rd;
@@ -126,6 +217,25 @@ __device__ __forceinline__ int UngappedWithTrigger(
   return sum;
 }
 
+// SeedSearcher::UngappedExtend as in ungapped.h, without reading ahead.
+__device__ __forceinline__ int UngappedByWord(const uint64_t *queries, uint32_t qpos,
+                                              const uint64_t *database, uint32_t dpos,
+                                              const PairTables<int8_t> &tables, int cutoff,
+                                              int trigger) {
+  const SeedWindow sq = LoadSeedWindow(queries, qpos), sd = LoadSeedWindow(database, dpos);
+  int sum = PairSideLazy<true>(queries, sq, database, sd, &tables, cutoff);
+  if (sum <= trigger) sum += PairSideLazy<false>(queries, sq, database, sd, &tables, cutoff);
+  return sum;
+}
+
+// Cutoffs in [1, kMaxByteCutoff] take the pair walk (ungapped.h), twelve
+// residues a step; the others, which its stop scores do not serve, go
+// residue by residue.  Bound: the issue of the walk's steps, a wave taking as
+// many as its longest seed on either side.  The grid is what the chip holds,
+// since a block's tables cost more to stage than a block's seeds to score.
+// 2,500,001 seeds of reads: 320 us residue by residue with blocks of 256
+// seeds, 164 us by pair steps that read ahead, 139 us without the read-ahead
+// (4 TB/s of fetched lines); 1,000 seeds 28 -> 6 us.
 __global__ void __launch_bounds__(256)
     UngappedTriggerKernel(size_t size, const uint32_t *qids,
                           const uint32_t *qpos, const uint32_t *dpos,
@@ -133,15 +243,27 @@ __global__ void __launch_bounds__(256)
                           const int *matrix, uint32_t nl, uint32_t delim,
                           const int *cutoffs, const int *triggers,
                           char *flags) {
+  __shared__ PairTables<int8_t> tables;
   __shared__ int8_t sm[kTableDim * kTableDim];
   StageScoreTable(sm, matrix, nl);
+  __syncthreads();
+  // the walk's tables: a delimiter stops, other codes past the matrix score 0
+  for (uint32_t i = threadIdx.x; i < kTableDim * kTableDim; i += blockDim.x) {
+    const uint32_t hi = i >> 5, lo = i & 31u;
+    const bool stop = hi == delim || lo == delim;
+    tables.ba[i] = stop ? (int8_t)kByteStopScore : sm[i];
+    tables.ab[i] = stop ? (int8_t)kByteStopScore : sm[lo * kTableDim + hi];
+  }
   __syncthreads();
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < size;
        i += (size_t)gridDim.x * blockDim.x) {
     const uint32_t q = qids[i];
-    const int trigger = triggers[q];
-    const int s = UngappedWithTrigger(queries, qpos[i], database, dpos[i], sm,
-                                      delim, cutoffs[q], trigger);
+    const int trigger = triggers[q], cutoff = cutoffs[q];
+    const int s = cutoff >= 1 && cutoff <= kMaxByteCutoff
+                      ? UngappedByWord(queries, qpos[i], database, dpos[i], tables, cutoff,
+                                       trigger)
+                      : UngappedByResidue(queries, qpos[i], database, dpos[i], sm, delim, cutoff,
+                                          trigger);
     flags[i] = (s > trigger) ? 1 : 0;
   }
 }
@@ -929,6 +1051,9 @@ inline unsigned Cus() {
   return (unsigned)cus;
 }
 
+// blocks of 256 threads that the chip holds at once (256 CUs, eight each)
+constexpr unsigned kResidentBlocks = 2048;
+
 inline unsigned GridFor(size_t n, unsigned block, unsigned cap = 65535u * 4) {
   size_t g = (n + block - 1) / block;
   if (g == 0) g = 1;
@@ -1104,7 +1229,12 @@ gz_status gz_distance_calculator_calculate_distances_async(
   hipStream_t s = S(stream);
   if (h_qc) GZ_HIP_CHECK(hipMemcpyAsync(d_qc, h_qc, size * 4, hipMemcpyDefault, s));
   if (h_dc) GZ_HIP_CHECK(hipMemcpyAsync(d_dc, h_dc, size * 4, hipMemcpyDefault, s));
-  hipLaunchKernelGGL(DistanceKernel, dim3(GridFor(size, 256)), dim3(256), 0, s,
+  // several pairs in flight per lane once every lane of the chip has several
+  const bool several = size > (size_t)kResidentBlocks * 256 * 2;
+  const auto kernel = h->length > kCodesPerWord ? DistanceKernel<1, true>
+                      : several                 ? DistanceKernel<4, false>
+                                                : DistanceKernel<1, false>;
+  hipLaunchKernelGGL(kernel, dim3(GridFor(size, 256, kResidentBlocks)), dim3(256), 0, s,
                      size, d_qc, d_dc, h->queries, h->database, h->reduced_map,
                      h->length, d_dist);
   GZ_HIP_CHECK(hipGetLastError());
@@ -1211,7 +1341,7 @@ gz_status gz_ungapped_extender_extend_with_trigger_async(
   if (h_qids) GZ_HIP_CHECK(hipMemcpyAsync(d_qids, h_qids, size * 4, hipMemcpyDefault, s));
   if (h_qpos) GZ_HIP_CHECK(hipMemcpyAsync(d_qpos, h_qpos, size * 4, hipMemcpyDefault, s));
   if (h_dpos) GZ_HIP_CHECK(hipMemcpyAsync(d_dpos, h_dpos, size * 4, hipMemcpyDefault, s));
-  hipLaunchKernelGGL(UngappedTriggerKernel, dim3(GridFor(size, 256)), dim3(256), 0,
+  hipLaunchKernelGGL(UngappedTriggerKernel, dim3(GridFor(size, 256, kResidentBlocks)), dim3(256), 0,
                      s, size, d_qids, d_qpos, d_dpos, h->queries, h->database,
                      h->matrix, h->number_letters, (uint32_t)h->delimiter,
                      h->cutoffs, h->triggers, d_flags);

@@ -43,13 +43,23 @@ struct SeedWindow {
   uint32_t k;
 };
 
+// Two neighbouring words in one read of 16 bytes.
+struct __attribute__((packed, aligned(8))) WordPair {
+  uint64_t lo, hi;
+};
+
+GZ_HD WordPair LoadWordPair(const uint64_t *p) {
+  return *reinterpret_cast<const WordPair *>(p);
+}
+
 GZ_HD SeedWindow LoadSeedWindow(const uint64_t *packed, uint32_t pos) {
   SeedWindow s;
   const uint32_t c = pos - kCodesPerWord + kPackPadCodes;
   s.wi = c / kCodesPerWord;
   s.k = c - s.wi * kCodesPerWord;
-  s.w0 = packed[s.wi] & kCodeBitsMask;
-  s.w1 = packed[s.wi + 1] & kCodeBitsMask;
+  const WordPair p = LoadWordPair(packed + s.wi);
+  s.w0 = p.lo & kCodeBitsMask;
+  s.w1 = p.hi & kCodeBitsMask;
   s.w2 = packed[s.wi + 2] & kCodeBitsMask;
   return s;
 }
@@ -166,13 +176,10 @@ GZ_HD PairWalk PairStart(const SeedWindow &sq, const SeedWindow &sd) {
   return w;
 }
 
-// Scores one window; false once the side has stopped (w.best is then its
-// score).
+// Scores the current window; false once the side has stopped (w.best is then
+// its score).
 template <bool kReverse, typename T>
-GZ_HD bool PairStep(const uint64_t *qw, const uint64_t *dw, const PairTables<T> *tab,
-                    int cutoff, PairWalk &w) {
-  const uint64_t qn = (kReverse ? qw[w.qi - 1] : qw[w.qi + 2]) & kCodeBitsMask;
-  const uint64_t dn = (kReverse ? dw[w.di - 1] : dw[w.di + 2]) & kCodeBitsMask;
+GZ_HD bool PairScore(const PairTables<T> *tab, int cutoff, PairWalk &w) {
   // Window12 of each pair; with k = 0 bits 60..63 hold stray bits, which no
   // field below reads
   const uint64_t Q = (w.q0 >> w.qr) | (w.q1 << w.ql);
@@ -195,8 +202,12 @@ GZ_HD bool PairStep(const uint64_t *qw, const uint64_t *dw, const PairTables<T> 
   }
   w.c = c;
   w.best = best;
-  // the pairs move on before the caller's exit test, so the read-ahead is
-  // used on every path and stays at the top of the step
+  return alive;
+}
+
+// Moves on by a window, qn and dn the words read.
+template <bool kReverse>
+GZ_HD void PairMove(uint64_t qn, uint64_t dn, PairWalk &w) {
   if (kReverse) {
     w.q1 = w.q0;
     w.q0 = qn;
@@ -212,6 +223,19 @@ GZ_HD bool PairStep(const uint64_t *qw, const uint64_t *dw, const PairTables<T> 
     ++w.qi;
     ++w.di;
   }
+}
+
+// Scores one window with the next word of each sequence read ahead; false
+// once the side has stopped.
+template <bool kReverse, typename T>
+GZ_HD bool PairStep(const uint64_t *qw, const uint64_t *dw, const PairTables<T> *tab,
+                    int cutoff, PairWalk &w) {
+  const uint64_t qn = (kReverse ? qw[w.qi - 1] : qw[w.qi + 2]) & kCodeBitsMask;
+  const uint64_t dn = (kReverse ? dw[w.di - 1] : dw[w.di + 2]) & kCodeBitsMask;
+  const bool alive = PairScore<kReverse>(tab, cutoff, w);
+  // the pairs move on before the caller's exit test, so the read-ahead is
+  // used on every path and stays at the top of the step
+  PairMove<kReverse>(qn, dn, w);
   return alive;
 }
 
@@ -241,6 +265,19 @@ GZ_HD int UngappedWithTrigger(const uint64_t *qw, uint32_t qpos, const uint64_t 
                               uint32_t dpos, const PairTables<T> *tab, int cutoff, int trigger) {
   const SeedWindow sq = LoadSeedWindow(qw, qpos), sd = LoadSeedWindow(dw, dpos);
   return UngappedWithTrigger(qw, sq, dw, sd, tab, cutoff, trigger);
+}
+
+// PairSide without the read-ahead: a word is read once a side goes on past
+// its window.  For callers bound by the number of scattered reads (most
+// sides stop in their first window).
+template <bool kReverse, typename T>
+GZ_HD int PairSideLazy(const uint64_t *qw, const SeedWindow &sq, const uint64_t *dw,
+                       const SeedWindow &sd, const PairTables<T> *tab, int cutoff) {
+  PairWalk w = PairStart<kReverse>(sq, sd);
+  while (PairScore<kReverse>(tab, cutoff, w))
+    PairMove<kReverse>((kReverse ? qw[w.qi - 1] : qw[w.qi + 2]) & kCodeBitsMask,
+                       (kReverse ? dw[w.di - 1] : dw[w.di + 2]) & kCodeBitsMask, w);
+  return w.best;
 }
 
 // Mismatches of the reduced codes over [qc - length/2, qc - length/2 +
