@@ -19,7 +19,7 @@ namespace gz {
 // allocation or free it makes mid-run hold this lock.
 std::recursive_mutex &CaptureLock();
 
-// Device workspaces of calls that have no handle to keep one.  A call takes a
+// Device workspaces of calls that keep none.  A call takes a
 // block, is its only user until its kernels and copies have ended, and gives
 // it back; one block per device is kept between calls, of at most kMost
 // bytes, the largest given back (a call that finds none, or one too small,

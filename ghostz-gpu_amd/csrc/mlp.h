@@ -52,32 +52,27 @@ class MlpDevice {
 
  private:
   hipError_t Reserve(size_t batch);
-  hipError_t ForwardDevice(size_t n, size_t padded);
-  hipError_t StepOnDevice(size_t n, size_t padded, float lr, long base, const uint32_t *done);
-  void SyncBf16();
+  hipError_t StepOnDevice(const uint8_t *codes, const float *targets, const uint32_t *order,
+                          size_t n, size_t padded, float lr, long step, float *loss, bool keep);
 
   hipError_t init_status_ = hipSuccess;
   hipStream_t stream_ = nullptr;
   size_t cap_ = 0;
-  // fp32 master weights + gradients + Adam moments, flat
+  void *weights_ = nullptr, *batch_ = nullptr;  // what the arrays below lie in
+  // fp32 master weights + gradients (the loss behind them) + Adam moments, flat
   float *master_ = nullptr, *grad_ = nullptr, *m_ = nullptr, *v_ = nullptr;
   uint16_t *w1h_ = nullptr, *w2h_ = nullptr, *embh_ = nullptr;  // bf16 copies
+  uint16_t *operands_ = nullptr;  // W1 and W2 as the training reads them, both ways
+  float *w1_parts_ = nullptr, *w2_parts_ = nullptr;  // weight gradients per slice of a batch
+  float *sums_ = nullptr;                            // other sums over a block's rows
   size_t count_ = 0;
   long step_ = 0;
   // activations
   uint8_t *codes_ = nullptr;
-  uint16_t *x_ = nullptr;       // [B][1024] bf16
-  float *z1_ = nullptr;         // [B][256]
   uint16_t *h1_ = nullptr;      // [B][256] bf16
-  float *z2_ = nullptr;         // [B][64]
-  uint16_t *h2_ = nullptr;      // [B][64] bf16
-  float *y_ = nullptr, *t_ = nullptr, *loss_ = nullptr;
-  float *dz2_ = nullptr;        // [B][64]
-  uint16_t *dz2h_ = nullptr;
-  float *dz1_ = nullptr;        // [B][256]
-  uint16_t *dz1h_ = nullptr;
-  float *dh1_ = nullptr;        // [B][256]
-  float *dx_ = nullptr;         // [B][1024]
+  float *t_ = nullptr;          // [B]
+  uint16_t *dz2h_ = nullptr;    // [B][64] bf16
+  uint16_t *dz1h_ = nullptr;    // [B][256] bf16
 };
 
 }  // namespace gz

@@ -1,10 +1,11 @@
 // mlp.hip -- see mlp.h.
 //
-// Every contraction runs through one bf16 MFMA GEMM kernel
-// (v_mfma_f32_32x32x8bf16_1k, fp32 accumulation): a 256-thread block owns a
-// 64 x 64 tile of C = A * B^T, each wave a 32 x 32 sub-tile; A and B are
-// addressed through (row, k) strides so the transposed products of the
-// backward pass reuse the same kernel.
+// A training step is three launches on bf16 MFMA with fp32 accumulation:
+// BatchKernel (forward, loss and the gradient down to the embeddings, 16 rows
+// of the batch per block), WeightGradKernel (what contracts over the batch)
+// and AdamKernel.  Sums over blocks go through stored partial sums: float
+// atomics of blocks on different XCDs meet in memory, 10 ns each on one
+// address.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -17,6 +18,7 @@
 #include "cost_model_gpu.h"
 #include "gz_runtime.h"
 #include "gz_common.h"
+#include "gz_device.h"
 #include "mlp.h"
 
 namespace gz {
@@ -51,277 +53,565 @@ __device__ __forceinline__ float GeluGrad(float z) {
   return cdf + z * pdf;
 }
 
-enum { kEpiStore = 0, kEpiBiasGelu = 1, kEpiGeluGrad = 2 };
-
-// C[m][n] = sum_k A(m, k) * B(n, k), A(m,k) = A[m*sam + k*sak], B likewise;
-// every operand has one unit stride (k for the forward and dX products, the
-// row for the weight gradients).  Blocks of four waves own 64 x 64 tiles of
-// C (32 x 32 per wave, v_mfma_f32_32x32x16_bf16); K advances 64 at a time
-// through LDS, where both operand tiles are stored k-contiguous, each filled
-// with 16-byte loads along the operand's unit stride; the next K slice is
-// read into registers while the current one is multiplied.  The weight
-// gradients have K = batch and few tiles: they split K over gridDim.z and
-// add their partial tiles into C (which the caller has zeroed).
-constexpr int kGemmTile = 64, kGemmK = 64, kGemmPad = 8;
 typedef __bf16 gemm_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float gemm_float4 __attribute__((ext_vector_type(4)));
 
-struct GemmSlice {
-  uint4 v[2];  // this thread's 16 values of one operand's 64 x 64 slice
+// ---------------------------------------------------------------------------
+// Training, first kernel: a block of four waves takes 16 rows of the batch
+// from their codes to the embedding gradient; layer inputs, pre-activations
+// and dX stay in registers and LDS.
+//
+// Tiles are v_mfma_f32_16x16x32_bf16: lane l supplies A[row l % 16][k] and
+// B[k][column l % 16] for k = 8 (l / 16) + j, j < 8; accumulator register r
+// holds C[4 (l / 16) + r][l % 16].  A wave owns 64 of the first layer's 256
+// units (four tiles), 16 of the second's 64, 256 of the 1024 inputs.  The
+// weights are kept once more in the order in which the lanes read them (a
+// tile's operand is 1 KB in a row; of the row-major weights it is 16 pieces
+// 2 KB apart) and
+// go from L2 straight into B operands, 16 of them ahead.  A operands of layer 1
+// are one residue's embedding each (kCostEmbed = 8), read by code from LDS.
+// Bound: a block's serial phases (one block per CU at 4,096 rows) and their
+// instruction fetches: a launch runs each line once or a few times, so that
+// loops unrolled into 40 KB of code took 77 us where these 10 KB take 41.
+// At 4,096 rows the work of this kernel took 160 us as 13 launches (embedding,
+// layers, output, loss, column sums, dZ2, dZ1, dX, embedding gradient).
+// ---------------------------------------------------------------------------
+constexpr int kRows = 16;        // of the batch per block
+constexpr int kTileK = 32;       // of one MFMA
+constexpr int kGroup = 4;        // k steps read together
+constexpr int kGroups = kCostIn / (kTileK * kGroup);
+constexpr int kWaveUnits = kCostH1 / 4;
+constexpr int kWaveTiles = kWaveUnits / 16;
+constexpr int kInputTiles = kCostIn / 4 / 16;  // of a wave
+constexpr int kH1Steps = kCostH1 / kTileK, kH2Steps = kCostH2 / kTileK;
+
+// Where operand value (column n, k) of a product over K values is kept.
+__device__ __forceinline__ size_t OperandAt(int n, int k, int K) {
+  return (size_t)(n / 16 * (K / kTileK) + k / kTileK) * (16 * kTileK) +
+         (n % 16 + k % kTileK / 8 * 16) * 8 + k % 8;
+}
+// This lane's part of the operand of columns 16 tile .. + 16, k step `step`.
+__device__ __forceinline__ gemm_bf16x8 Operand(const uint16_t *p, int tile, int step, int K) {
+  return *reinterpret_cast<const gemm_bf16x8 *>(
+      p + (size_t)(tile * (K / kTileK) + step) * (16 * kTileK) + (threadIdx.x & 63) * 8);
+}
+
+// The weights in operand order: W1 by unit (k: inputs) and by input (k:
+// units), W2 by unit and by hidden unit.
+struct Operands {
+  uint16_t *w1, *w1t, *w2, *w2t;
 };
 
-// Thread t's part of the slice of rows [r0, r0 + 64) x k [k0, k0 + 64):
-// with unit k stride, row r0 + t / 4 and k's (t % 4) * 16 .. + 16; with unit
-// row stride, k0 + t / 4 and rows (t % 4) * 16 .. + 16.  Out-of-range values
-// read 0.
-template <bool kUnitK>
-__device__ __forceinline__ void GemmLoadSlice(GemmSlice &g, const uint16_t *X, long sr, long sk,
-                                              int rows, int K, int r0, int k0) {
-  const int t = threadIdx.x;
-  const int a = t >> 2, b = (t & 3) * 16;
-  const int gr = kUnitK ? r0 + a : r0 + b, gk = kUnitK ? k0 + b : k0 + a;
-  const uint16_t *p = X + (long)gr * sr + (long)gk * sk;
-  const bool fast = kUnitK ? (gr < rows && gk + 16 <= K) : (gk < K && gr + 16 <= rows);
-  if (fast && ((reinterpret_cast<uintptr_t>(p) & 15) == 0)) {
-    g.v[0] = *reinterpret_cast<const uint4 *>(p);
-    g.v[1] = *reinterpret_cast<const uint4 *>(p + 8);
-  } else {
-    uint16_t h[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int rr = kUnitK ? gr : gr + j, kk = kUnitK ? gk + j : gk;
-      h[j] = (rr < rows && kk < K) ? X[(long)rr * sr + (long)kk * sk] : (uint16_t)0;
-    }
-    memcpy(&g.v[0], h, 32);
-  }
-}
+static_assert(kOffW3 == kOffB2 + kCostH2 && kOffB3 == kOffW3 + kCostH2, "sums in weight order");
+static_assert(kCostEmbed == 8 && kCostH1 == 256 && kCostH2 == 64, "the block's tiles");
 
-template <bool kUnitK>
-__device__ __forceinline__ void GemmStoreSlice(uint16_t (*T)[kGemmK + kGemmPad],
-                                               const GemmSlice &g) {
-  const int t = threadIdx.x;
-  const int a = t >> 2, b = (t & 3) * 16;
-  if (kUnitK) {
-    *reinterpret_cast<uint4 *>(&T[a][b]) = g.v[0];
-    *reinterpret_cast<uint4 *>(&T[a][b + 8]) = g.v[1];
-  } else {
-    uint16_t h[16];
-    memcpy(h, &g.v[0], 32);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) T[b + j][a] = h[j];
-  }
-}
+// The batch's rows: row r < n is row order[r] (r without order) of codes and
+// targets; rows past n read code 20 and count nothing.
+struct BatchRows {
+  const uint8_t *codes;
+  const float *targets;
+  const uint32_t *order;
+  int n;
+};
 
-template <int EPI, bool kUnitKA, bool kUnitKB>
-__global__ void __launch_bounds__(256)
-    GemmKernel(int M, int N, int K, const uint16_t *A, long sam, long sak,
-               const uint16_t *B, long sbn, long sbk, float *C, int ldc,
-               const float *bias, uint16_t *Ch, const float *zsaved) {
-  __shared__ __align__(16) uint16_t As[kGemmTile][kGemmK + kGemmPad];
-  __shared__ __align__(16) uint16_t Bs[kGemmTile][kGemmK + kGemmPad];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int mb = blockIdx.y * kGemmTile, nb = blockIdx.x * kGemmTile;
-  const int m0 = mb + (wave >> 1) * 32, n0 = nb + (wave & 1) * 32;
-  const int am = (wave >> 1) * 32 + (lane & 31), bn = (wave & 1) * 32 + (lane & 31);
-  const int kq = (lane >> 5) * 8;
-  // this block's K range (split K: gridDim.z slices of whole 64-steps)
-  const int steps = (K + kGemmK - 1) / kGemmK;
-  const int per = (steps + (int)gridDim.z - 1) / (int)gridDim.z;
-  const int kb = (int)blockIdx.z * per * kGemmK, ke = min(K, kb + per * kGemmK);
-  float16_t acc;
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  GemmSlice ga, gb;
-  if (kb < ke) {
-    GemmLoadSlice<kUnitKA>(ga, A, sam, sak, M, ke, mb, kb);
-    GemmLoadSlice<kUnitKB>(gb, B, sbn, sbk, N, ke, nb, kb);
-  }
-  for (int k0 = kb; k0 < ke; k0 += kGemmK) {
-    GemmStoreSlice<kUnitKA>(As, ga);
-    GemmStoreSlice<kUnitKB>(Bs, gb);
-    __syncthreads();
-    if (k0 + kGemmK < ke) {  // the next slice's loads overlap this slice's MFMAs
-      GemmLoadSlice<kUnitKA>(ga, A, sam, sak, M, ke, mb, k0 + kGemmK);
-      GemmLoadSlice<kUnitKB>(gb, B, sbn, sbk, N, ke, nb, k0 + kGemmK);
-    }
+// A block's sums over its rows: the gradients of the embedding, of the biases
+// and of the output weights, and the loss.
+constexpr int kSumB1 = kCostAlphabet * kCostEmbed, kSumB2 = kSumB1 + kCostH1,
+              kSumW3 = kSumB2 + kCostH2, kSumB3 = kSumW3 + kCostH2, kSumLoss = kSumB3 + 1,
+              kSums = kSumLoss + 1;
+constexpr int kMostBatchBlocks = 1024;
+
+__global__ void __launch_bounds__(256, 1)
+    BatchKernel(BatchRows rows, int tiles, const uint16_t *embh, Operands weights,
+                const float *b1, const float *b2, const float *w3, const float *b3,
+                uint8_t *batch_codes, uint16_t *h1, uint16_t *dz2h, uint16_t *dz1h, float *sums) {
+  constexpr int kPad = 8;
+  __shared__ uint4 emb[kCostAlphabet];
+  __shared__ __align__(16) uint32_t codes[kRows][kCostResidues / 4 + 1];
+  __shared__ __align__(16) uint16_t tile[kRows][kCostH1 + kPad];  // h1, then dz1
+  __shared__ __align__(16) uint16_t dz2t[kRows][kCostH2 + kPad];
+  __shared__ float z1t[kRows][kCostH1 + 4], dh1t[kRows][kCostH1 + 4];
+  __shared__ float zt[kRows][kCostH2 + 1], pt[kRows][kCostH2 + 1];
+  __shared__ float w3s[kCostH2];
+  __shared__ float part[2][4];
+  __shared__ float table[kCostAlphabet * kCostEmbed];
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  const int l16 = lane & 15, quarter = lane >> 4;
+  const int hr = t >> 4;  // the row of 16 threads
+  const float bias1 = b1[t], bias2 = b2[wave * 16 + l16], bias3 = b3[0];
+  if (t < kCostAlphabet) emb[t] = reinterpret_cast<const uint4 *>(embh)[t];
+  if (t < kCostAlphabet * kCostEmbed) table[t] = 0.f;
+  if (t < kCostH2) w3s[t] = Bf2F(F2Bf(w3[t]));
+  float sum1 = 0.f, sum2 = 0.f;  // of unit t's dZ1, and of what thread t sums below
+  for (int row_tile = blockIdx.x; row_tile < tiles; row_tile += gridDim.x) {
+    const int base = row_tile * kRows;
+    // layer 1's weights: group g's operand of k step s and tile i
+    gemm_bf16x8 w[2][kGroup][kWaveTiles];
+    auto read_group = [&](int g, gemm_bf16x8 (&v)[kGroup][kWaveTiles]) {
 #pragma unroll
-    for (int ks = 0; ks < kGemmK; ks += 16) {
-      const gemm_bf16x8 a = *reinterpret_cast<const gemm_bf16x8 *>(&As[am][ks + kq]);
-      const gemm_bf16x8 b = *reinterpret_cast<const gemm_bf16x8 *>(&Bs[bn][ks + kq]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    }
-    __syncthreads();
-  }
+      for (int i = 0; i < kWaveTiles; ++i)
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int row = m0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-    const int col = n0 + (lane & 31);
-    if (row < M && col < N) {
-      const long idx = (long)row * ldc + col;
-      const float v = acc[r];
-      if (EPI == kEpiStore) {
-        if (gridDim.z > 1) atomicAdd(&C[idx], v);
-        else C[idx] = v;
-      } else if (EPI == kEpiBiasGelu) {
-        const float z = v + bias[col];
-        C[idx] = z;
-        Ch[idx] = F2Bf(Gelu(z));
-      } else {
-        const float dz = v * GeluGrad(zsaved[idx]);
-        C[idx] = dz;
-        Ch[idx] = F2Bf(dz);
+        for (int s = 0; s < kGroup; ++s)
+          v[s][i] = Operand(weights.w1, wave * kWaveTiles + i, g * kGroup + s, kCostIn);
+    };
+    // the rows' codes, 16 threads of eight each
+    float target = 0.f;
+    {
+      const int b = base + hr, k = (t & 15) * 2;
+      uint2 c = make_uint2(0x14141414u, 0x14141414u);
+      if (b < rows.n) {
+        const size_t at = rows.order ? rows.order[b] : (uint32_t)b;
+        c = *reinterpret_cast<const uint2 *>(rows.codes + at * kCostResidues + k * 4);
+        target = rows.targets[at];
+      }
+      codes[hr][k] = c.x;
+      codes[hr][k + 1] = c.y;
+      *reinterpret_cast<uint2 *>(batch_codes + (size_t)b * kCostResidues + k * 4) = c;
+    }
+    read_group(0, w[0]);
+    __syncthreads();
+    gemm_float4 acc[kWaveTiles];
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; ++i) acc[i] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int g0 = 0; g0 < kGroups; g0 += 2) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int g = g0 + h;
+        read_group(g + 1 < kGroups ? g + 1 : g, w[h ^ 1]);  // (the last one again)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < kGroup; ++s) {
+          // residue 4 (g kGroup + s) + quarter of the lane's row
+          const uint32_t c = (codes[l16][g * kGroup + s] >> (8 * quarter)) & 0xffu;
+          const gemm_bf16x8 a = *reinterpret_cast<const gemm_bf16x8 *>(
+              &emb[c < (uint32_t)kCostAlphabet ? c : kCostAlphabet - 1]);
+#pragma unroll
+          for (int i = 0; i < kWaveTiles; ++i)
+            acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w[h][s][i], acc[i], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-  }
-}
-
-__global__ void EmbedKernel(int B, const uint8_t *codes, const uint16_t *embh, uint16_t *x) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long)B * kCostIn) return;
-  const long b = i / kCostIn;
-  const int c = (int)(i % kCostIn);
-  const int r = c / kCostEmbed, e = c % kCostEmbed;
-  const int a = min((int)codes[b * kCostResidues + r], kCostAlphabet - 1);
-  x[i] = embh[a * kCostEmbed + e];
-}
-
-__global__ void OutputKernel(int B, const uint16_t *h2, const float *w3, const float *b3,
-                             float *y) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  float s = 0.f;
-  for (int k = 0; k < kCostH2; ++k) s += Bf2F(h2[b * kCostH2 + k]) * Bf2F(F2Bf(w3[k]));
-  y[b] = s + b3[0];
-}
-
-// Batch rows from a device-resident training set: row r < n of step *done
-// is row order_base[*done * n + r] of (codes, targets); padding rows read
-// code 20 and target 0.  One thread per 16 bytes of the batch's codes.
-__global__ void GatherRowsKernel(const uint8_t *codes, const float *targets,
-                                 const uint32_t *order_base, const uint32_t *done, int n, int B,
-                                 uint8_t *out_codes, float *out_t) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  constexpr int kPieces = kCostResidues / 16;
-  if (i >= B * kPieces) return;
-  // the batch of step *done
-  const uint32_t *order = order_base + (size_t)*done * (size_t)n;
-  const int r = i / kPieces, k = i % kPieces;
-  uint4 v = make_uint4(0x14141414u, 0x14141414u, 0x14141414u, 0x14141414u);
-  if (r < n) v = reinterpret_cast<const uint4 *>(codes + (size_t)order[r] * kCostResidues)[k];
-  reinterpret_cast<uint4 *>(out_codes + (size_t)r * kCostResidues)[k] = v;
-  if (k == 0) out_t[r] = r < n ? targets[order[r]] : 0.f;
-}
-
-// End of a step: its loss into the sum, the step count up by one.
-__global__ void AdvanceKernel(const float *loss, float *sum, uint32_t *done) {
-  if (threadIdx.x == 0) {
-    *sum += *loss;
-    *done += 1;
-  }
-}
-
-// MSE loss over the first n rows; dY = 2 (y - t) / n, zero on padding.
-__global__ void LossKernel(int B, int n, const float *y, const float *t, float *dy,
-                           float *loss) {
-  __shared__ float part[256];
-  float acc = 0.f;
-  for (int b = threadIdx.x; b < B; b += blockDim.x) {
-    float g = 0.f;
-    if (b < n) {
-      const float d = y[b] - t[b];
-      acc += d * d;
-      g = 2.f * d / n;
-    }
-    dy[b] = g;
-  }
-  part[threadIdx.x] = acc;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) part[threadIdx.x] += part[threadIdx.x + s];
+    // the second layer's operands, in flight during the GELUs
+    gemm_bf16x8 v2[kH1Steps], vt[kH2Steps][kWaveTiles];
+#pragma unroll
+    for (int s = 0; s < kH1Steps; ++s) v2[s] = Operand(weights.w2, wave, s, kCostH1);
+#pragma unroll
+    for (int s = 0; s < kH2Steps; ++s)
+#pragma unroll
+      for (int i = 0; i < kWaveTiles; ++i)
+        vt[s][i] = Operand(weights.w2t, wave * kWaveTiles + i, s, kCostH2);
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        z1t[4 * quarter + r][wave * kWaveUnits + i * 16 + l16] = acc[i][r];
     __syncthreads();
-  }
-  if (threadIdx.x == 0) loss[0] = part[0] / n;
-}
-
-// dZ2 = dY w3 * gelu'(Z2), elementwise over B x 64
-__global__ void OutputBackwardKernel(int B, const float *dy, const float *z2, const float *w3,
-                                     float *dz2, uint16_t *dz2h) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= B * kCostH2) return;
-  const int b = i / kCostH2, k = i % kCostH2;
-  const float d = dy[b] * Bf2F(F2Bf(w3[k])) * GeluGrad(z2[i]);
-  dz2[i] = d;
-  dz2h[i] = F2Bf(d);
-}
-
-// out[c] += sum_b wt[b] * M[b][c] (wt optional); M is fp32 or bf16.  Blocks
-// own 64 columns and a slice of rows; partial sums are added atomically.
-template <typename T>
-__global__ void __launch_bounds__(256)
-    ColumnSumKernel(int B, int N, const T *m, const float *wt, float *out) {
-  __shared__ float part[4][64];
-  const int c = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int lane_row = threadIdx.x >> 6;
-  const int rows = (B + gridDim.y - 1) / gridDim.y;
-  const int r0 = blockIdx.y * rows, r1 = min(B, r0 + rows);
-  float s = 0.f;
-  if (c < N)
-    for (int b = r0 + lane_row; b < r1; b += 4) {
-      float v;
-      if constexpr (sizeof(T) == 2) v = Bf2F((uint16_t)m[(long)b * N + c]);
-      else v = (float)m[(long)b * N + c];
-      s += wt ? wt[b] * v : v;
+    // z1 and h1, a unit per thread
+#pragma unroll 2
+    for (int r = 0; r < kRows; ++r) {
+      const float z = z1t[r][t] + bias1;
+      z1t[r][t] = z;
+      tile[r][t] = F2Bf(Gelu(z));
     }
-  part[lane_row][threadIdx.x & 63] = s;
-  __syncthreads();
-  if (threadIdx.x < 64 && c < N)
-    atomicAdd(&out[c], part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] +
-                           part[3][threadIdx.x]);
-}
-
-// d_embed[a][e] = sum over (b, r) with code a of dX[b][r*8 + e]
-__global__ void EmbedBackwardKernel(int B, const uint8_t *codes, const float *dx, float *gemb) {
-  __shared__ float acc[kCostAlphabet * kCostEmbed];
-  for (int i = threadIdx.x; i < kCostAlphabet * kCostEmbed; i += blockDim.x) acc[i] = 0.f;
-  __syncthreads();
-  const long total = (long)B * kCostIn;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (long)gridDim.x * blockDim.x) {
-    const long b = i / kCostIn;
-    const int c = (int)(i % kCostIn);
-    const int a = min((int)codes[b * kCostResidues + c / kCostEmbed], kCostAlphabet - 1);
-    atomicAdd(&acc[a * kCostEmbed + c % kCostEmbed], dx[i]);
+    __syncthreads();
+    auto store_tile = [&](uint16_t *out) {  // 16 threads per row, 16 values each
+      const int c = (t & 15) * 16;
+      uint4 *o = reinterpret_cast<uint4 *>(out + (size_t)(base + hr) * kCostH1 + c);
+      const uint4 *x = reinterpret_cast<const uint4 *>(&tile[hr][c]);
+      o[0] = x[0];
+      o[1] = x[1];
+    };
+    store_tile(h1);
+    {
+      gemm_float4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < kH1Steps; ++s)
+        z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            *reinterpret_cast<const gemm_bf16x8 *>(&tile[l16][s * kTileK + 8 * quarter]), v2[s],
+            z, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) zt[4 * quarter + r][wave * 16 + l16] = z[r] + bias2;
+    }
+    __syncthreads();
+    // the head, 16 threads per row and four units each: output, mean squared
+    // error and its gradient, dZ2 = dY w3 * gelu'(Z2)
+    {
+      const int c0 = (t & 15) * 4, b = base + hr;
+      float s = 0.f;
+#pragma unroll 1
+      for (int c = c0; c < c0 + 4; ++c) {
+        const float h = Bf2F(F2Bf(Gelu(zt[hr][c])));
+        pt[hr][c] = h;
+        s += h * w3s[c];
+      }
+#pragma unroll
+      for (int m = 1; m < 16; m <<= 1) s += __shfl_xor(s, m, kWave);
+      const float d = b < rows.n ? s + bias3 - target : 0.f;
+      const float dy = 2.f * d / rows.n;
+#pragma unroll 1
+      for (int c = c0; c < c0 + 4; ++c) {
+        const float dz = dy * w3s[c] * GeluGrad(zt[hr][c]);
+        zt[hr][c] = dz;
+        pt[hr][c] *= dy;
+        dz2t[hr][c] = F2Bf(dz);
+      }
+      *reinterpret_cast<uint2 *>(dz2h + (size_t)b * kCostH2 + c0) =
+          *reinterpret_cast<const uint2 *>(&dz2t[hr][c0]);
+      float e = d * d, g = dy;
+      e += __shfl_xor(e, 16, kWave);
+      g += __shfl_xor(g, 16, kWave);
+      e += __shfl_xor(e, 32, kWave);
+      g += __shfl_xor(g, 32, kWave);
+      if (lane == 0) {
+        part[0][wave] = g;
+        part[1][wave] = e;
+      }
+    }
+    __syncthreads();
+    // dB2 = sum dZ2, dW3 = H2^T dY, dB3 = sum dY and the loss
+    if (t < 2 * kCostH2) {
+      const int c = t & (kCostH2 - 1);
+      const float(*m)[kCostH2 + 1] = t < kCostH2 ? zt : pt;
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) sum2 += m[r][c];
+    } else if (t < 2 * kCostH2 + 2) {
+      const float *p = part[t & 1];
+      const float sum = (p[0] + p[1]) + (p[2] + p[3]);
+      sum2 += t & 1 ? sum / rows.n : sum;
+    }
+    // dZ1 = (dZ2 W2) * gelu'(Z1) and dB1 = sum dZ1; the h1 tile is read out
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; ++i) {
+      gemm_float4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < kH2Steps; ++s)
+        z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            *reinterpret_cast<const gemm_bf16x8 *>(&dz2t[l16][s * kTileK + 8 * quarter]),
+            vt[s][i], z, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        dh1t[4 * quarter + r][wave * kWaveUnits + i * 16 + l16] = z[r];
+    }
+    // dX = dZ1 W1, a wave's 256 inputs two tiles at a time
+    constexpr int kPairsOfTiles = kInputTiles / 2;
+    gemm_bf16x8 u[2][2][kH1Steps];
+    auto read_inputs = [&](int p, gemm_bf16x8 (&v)[2][kH1Steps]) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int s = 0; s < kH1Steps; ++s)
+          v[i][s] = Operand(weights.w1t, wave * kInputTiles + 2 * p + i, s, kCostH1);
+    };
+    read_inputs(0, u[0]);
+    __syncthreads();
+#pragma unroll 2
+    for (int r = 0; r < kRows; ++r) {
+      const float dz = dh1t[r][t] * GeluGrad(z1t[r][t]);
+      sum1 += dz;
+      tile[r][t] = F2Bf(dz);
+    }
+    __syncthreads();
+    store_tile(dz1h);
+    gemm_bf16x8 dz[kH1Steps];
+#pragma unroll
+    for (int s = 0; s < kH1Steps; ++s)
+      dz[s] = *reinterpret_cast<const gemm_bf16x8 *>(&tile[l16][s * kTileK + 8 * quarter]);
+#pragma unroll 1
+    for (int p0 = 0; p0 < kPairsOfTiles; p0 += 2) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int p = p0 + h;
+        read_inputs(p + 1 < kPairsOfTiles ? p + 1 : p, u[h ^ 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        gemm_float4 x[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          x[i] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int s = 0; s < kH1Steps; ++s)
+            x[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dz[s], u[h][i][s], x[i], 0, 0, 0);
+        }
+        // the embedding gradient: the sum over (row, residue) with code a of
+        // the residue's eight columns; a tile is two residues
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int residue = (wave * kInputTiles + 2 * p + i) * 2 + (l16 >> 3);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const uint32_t c =
+                (codes[4 * quarter + r][residue >> 2] >> (8 * (residue & 3))) & 0xffu;
+            atomicAdd(&table[(c < (uint32_t)kCostAlphabet ? c : kCostAlphabet - 1) * kCostEmbed +
+                             (l16 & 7)],
+                      x[i][r]);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();  // the tile, the codes and the table are read or written
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < kCostAlphabet * kCostEmbed; i += blockDim.x)
-    atomicAdd(&gemb[i], acc[i]);
+  float *out = sums + (size_t)blockIdx.x * kSums;
+  if (t < kCostAlphabet * kCostEmbed) out[t] = table[t];
+  out[kSumB1 + t] = sum1;
+  if (t < 2 * kCostH2 + 2) out[kSumB2 + t] = sum2;  // dB2, dW3, dB3, the loss
 }
 
-__global__ void AdamKernel(size_t n, float *w, const float *g, float *m, float *v, float lr,
-                           float b1, float b2, float c1, float c2, float eps) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+// ---------------------------------------------------------------------------
+// Training, second kernel: products over 64 x 64 tiles of C[m][n] =
+// sum_k A(m, k) B(n, k), a 32 x 32 part per wave (v_mfma_f32_32x32x16_bf16).
+// K advances 128 at a time through LDS, where both operand tiles are stored
+// k-contiguous; the next two slices are on their way into registers while the
+// current one is multiplied.  Sizes are multiples of 64 and rows 16-byte
+// aligned.  Values from ke on read 0.
+// ---------------------------------------------------------------------------
+constexpr int kGemmTile = 64, kGemmK = 128, kGemmPad = 8;
+typedef uint16_t GemmLdsTile[kGemmTile][kGemmK + kGemmPad];
+
+// Transposes the k pairs t / 8 + 32 i of rows (t % 8) * 8 .. + 8, v[2 i] the
+// even k's values and v[2 i + 1] the odd one's.
+__device__ __forceinline__ void StorePairs(GemmLdsTile &T, const uint4 (&v)[4]) {
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    uint16_t lo[8], hi[8];
+    memcpy(lo, &v[2 * i], 16);
+    memcpy(hi, &v[2 * i + 1], 16);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      *reinterpret_cast<uint32_t *>(&T[(t & 7) * 8 + j][2 * ((t >> 3) + 32 * i)]) =
+          (uint32_t)lo[j] | (uint32_t)hi[j] << 16;
+  }
 }
 
-// Adam with the step number on the device: t = base + *done + 1 (a step
-// sequence replayed from a graph keeps its own count).
-__global__ void AdamCountedKernel(size_t n, float *w, const float *g, float *m, float *v,
-                                  float lr, float b1, float b2, float eps, long base,
-                                  const uint32_t *done) {
+// An operand with unit row stride.
+struct ColumnOperand {
+  const uint16_t *p;
+  long stride;
+  struct Slice {
+    uint4 v[4];
+  };
+  __device__ __forceinline__ void Load(Slice &g, int r0, int k0, int ke) const {
+    const int t = threadIdx.x;
+    const uint16_t *x = p + r0 + (t & 7) * 8;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int k = k0 + 2 * ((t >> 3) + 32 * (i >> 1)) + (i & 1);
+      g.v[i] = k < ke ? *reinterpret_cast<const uint4 *>(x + k * stride) : make_uint4(0, 0, 0, 0);
+    }
+  }
+  __device__ __forceinline__ void Store(GemmLdsTile &T, const Slice &g) const {
+    StorePairs(T, g.v);
+  }
+};
+
+// The batch's embeddings as such an operand: eight rows are one residue.
+struct EmbedOperand {
+  const uint8_t *codes;
+  const uint4 *emb;  // in LDS, zeros behind the alphabet
+  struct Slice {
+    uint8_t c[4];
+  };
+  __device__ __forceinline__ void Load(Slice &g, int r0, int k0, int ke) const {
+    const int t = threadIdx.x;
+    const uint8_t *x = codes + r0 / kCostEmbed + (t & 7);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int k = k0 + 2 * ((t >> 3) + 32 * (i >> 1)) + (i & 1);
+      uint8_t c = kCostAlphabet;
+      if (k < ke) {
+        c = x[(size_t)k * kCostResidues];
+        c = c < kCostAlphabet ? c : (uint8_t)(kCostAlphabet - 1);
+      }
+      g.c[i] = c;
+    }
+  }
+  __device__ __forceinline__ void Store(GemmLdsTile &T, const Slice &g) const {
+    uint4 v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = emb[g.c[i]];
+    StorePairs(T, v);
+  }
+};
+
+struct GemmLds {
+  __align__(16) GemmLdsTile a;
+  __align__(16) GemmLdsTile b;
+};
+
+// The wave's 32 x 32 part of the tile at (mb, nb) over k [kb, ke).
+template <class A, class B>
+__device__ __forceinline__ float16_t GemmTile(GemmLds &T, const A &x, const B &y, int mb, int nb,
+                                              int kb, int ke) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int am = (wave >> 1) * 32 + (lane & 31), bn = (wave & 1) * 32 + (lane & 31);
+  const int kq = (lane >> 5) * 8;
+  float16_t acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  typename A::Slice ga[2];
+  typename B::Slice gb[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    x.Load(ga[h], mb, kb + h * kGemmK, ke);
+    y.Load(gb[h], nb, kb + h * kGemmK, ke);
+  }
+  for (int k0 = kb; k0 < ke; k0 += 2 * kGemmK) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (k0 + h * kGemmK >= ke) break;
+      x.Store(T.a, ga[h]);
+      y.Store(T.b, gb[h]);
+      __syncthreads();
+      x.Load(ga[h], mb, k0 + (h + 2) * kGemmK, ke);
+      y.Load(gb[h], nb, k0 + (h + 2) * kGemmK, ke);
+#pragma unroll
+      for (int ks = 0; ks < kGemmK; ks += 16) {
+        const gemm_bf16x8 a = *reinterpret_cast<const gemm_bf16x8 *>(&T.a[am][ks + kq]);
+        const gemm_bf16x8 b = *reinterpret_cast<const gemm_bf16x8 *>(&T.b[bn][ks + kq]);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+      }
+      __syncthreads();
+    }
+  }
+  return acc;
+}
+
+// Row and column inside the tile of accumulator register r of this thread.
+__device__ __forceinline__ int TileRow(int r) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  return (wave >> 1) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+}
+__device__ __forceinline__ int TileCol() {
+  return ((threadIdx.x >> 6) & 1) * 32 + (threadIdx.x & 31);
+}
+
+// The batch's slices that the two weight gradients are split into.
+struct BatchSplit {
+  int w1_slices, w1_rows, w2_slices, w2_rows;  // slices, rows of the batch each
+};
+constexpr int kW1Tiles = (kCostH1 / kGemmTile) * (kCostIn / kGemmTile);
+constexpr int kW2Tiles = kCostH1 / kGemmTile;
+constexpr int kMostW1Slices = 8, kMostW2Slices = 32;
+
+// The two weight gradients in one launch: blocks [0, w1) dW1 = dZ1^T X, 64
+// tiles times its slices, the others dW2 = dZ2^T H1, 4 tiles times its
+// slices, both as partial gradients per slice; then the blocks' sums of the
+// first kernel, 64 values a block.  Bound: the latency of a block's four
+// slices of K and the barriers between them; 17 us at 4,096 rows, where the
+// two products took 45 us with the partial tiles added by atomics.
+__global__ void __launch_bounds__(256)
+    WeightGradKernel(int B, BatchSplit split, const uint16_t *h1, const uint16_t *dz1h,
+                     const uint16_t *dz2h, const uint8_t *codes, const uint16_t *embh,
+                     float *w1_parts, float *w2_parts, const float *sums, int nsums, float *grad,
+                     float *loss) {
+  __shared__ GemmLds T;
+  __shared__ uint4 emb[kCostAlphabet + 1];
+  int block = blockIdx.x;
+  const int w1 = kW1Tiles * split.w1_slices;
+  auto store = [&](float *c, int cols, int mb, int nb, const float16_t &acc) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      c[(size_t)(mb + TileRow(r)) * cols + nb + TileCol()] = acc[r];
+  };
+  if (block < w1) {
+    if (threadIdx.x <= kCostAlphabet)
+      emb[threadIdx.x] = threadIdx.x < kCostAlphabet
+                             ? reinterpret_cast<const uint4 *>(embh)[threadIdx.x]
+                             : make_uint4(0, 0, 0, 0);
+    __syncthreads();
+    const int tile = block % kW1Tiles, slice = block / kW1Tiles;
+    const int mb = tile / (kCostIn / kGemmTile) * kGemmTile,
+              nb = tile % (kCostIn / kGemmTile) * kGemmTile;
+    const int kb = slice * split.w1_rows, ke = min(B, kb + split.w1_rows);
+    store(w1_parts + (size_t)slice * kCostH1 * kCostIn, kCostIn, mb, nb,
+          GemmTile(T, ColumnOperand{dz1h, kCostH1}, EmbedOperand{codes, emb}, mb, nb, kb, ke));
+    return;
+  }
+  block -= w1;
+  if (block >= kW2Tiles * split.w2_slices) {
+    __shared__ float part[3][64];
+    const int c = (block - kW2Tiles * split.w2_slices) * 64 + (int)(threadIdx.x & 63);
+    const int wave = threadIdx.x >> 6;
+    float sum = 0.f;
+    if (c < kSums) {
+#pragma unroll 16
+      for (int b = wave; b < nsums; b += 4) sum += sums[(size_t)b * kSums + c];
+    }
+    if (wave > 0) part[wave - 1][threadIdx.x & 63] = sum;
+    __syncthreads();
+    if (wave > 0 || c >= kSums) return;
+    sum += (part[0][threadIdx.x] + part[1][threadIdx.x]) + part[2][threadIdx.x];
+    if (c < kSumB1) grad[kOffEmbed + c] = sum;
+    else if (c < kSumB2) grad[kOffB1 + c - kSumB1] = sum;
+    else if (c < kSumLoss) grad[kOffB2 + c - kSumB2] = sum;
+    else *loss += sum;
+    return;
+  }
+  const int nb = block % kW2Tiles * kGemmTile, slice = block / kW2Tiles;
+  const int kb = slice * split.w2_rows, ke = min(B, kb + split.w2_rows);
+  store(w2_parts + (size_t)slice * kCostH2 * kCostH1, kCostH1, 0, nb,
+        GemmTile(T, ColumnOperand{dz2h, kCostH2}, ColumnOperand{h1, kCostH1}, 0, nb, kb, ke));
+}
+
+// ---------------------------------------------------------------------------
+// Training, third kernel: the gradient's partial sums, Adam and the bf16
+// copies of the weights.
+// ---------------------------------------------------------------------------
+struct Adam {
+  float *w, *m, *v;
+  uint16_t *w1h, *w2h, *embh;
+  Operands o;
+  float lr, b1, b2, eps;
+  // weight i's bf16 copies
+  __device__ __forceinline__ void Copy(size_t i, float x) const {
+    const uint16_t h = F2Bf(x);
+    if (i < kOffW1) {
+      embh[i] = h;
+    } else if (i < kOffB1) {
+      const int k = (int)(i - kOffW1), unit = k / kCostIn, in = k % kCostIn;
+      w1h[k] = h;
+      o.w1[OperandAt(unit, in, kCostIn)] = h;
+      o.w1t[OperandAt(in, unit, kCostH1)] = h;
+    } else if (i >= kOffW2 && i < kOffB2) {
+      const int k = (int)(i - kOffW2), unit = k / kCostH1, hidden = k % kCostH1;
+      w2h[k] = h;
+      o.w2[OperandAt(unit, hidden, kCostH1)] = h;
+      o.w2t[OperandAt(hidden, unit, kCostH2)] = h;
+    }
+  }
+};
+
+// c1, c2: the step's bias corrections; lr = 0: no update.  keep: the whole
+// gradient is left in g (W1's and W2's are only summed here).
+__global__ void __launch_bounds__(256)
+    AdamKernel(size_t n, Adam a, float *g, BatchSplit split, const float *w1_parts,
+               const float *w2_parts, float c1, float c2, int keep) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const float t = (float)(base + (long)*done + 1);
-  const float c1 = 1.f - powf(b1, t), c2 = 1.f - powf(b2, t);
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  float gi;
+  if (i >= kOffW1 && i < kOffB1) {
+    gi = 0.f;
+    for (int k = 0; k < split.w1_slices; ++k)
+      gi += w1_parts[(size_t)k * kCostH1 * kCostIn + (i - kOffW1)];
+    if (keep) g[i] = gi;
+  } else if (i >= kOffW2 && i < kOffB2) {
+    gi = 0.f;
+    for (int k = 0; k < split.w2_slices; ++k)
+      gi += w2_parts[(size_t)k * kCostH2 * kCostH1 + (i - kOffW2)];
+    if (keep) g[i] = gi;
+  } else {
+    gi = g[i];
+  }
+  if (a.lr == 0.f) return;
+  const float mi = a.b1 * a.m[i] + (1.f - a.b1) * gi;
+  const float vi = a.b2 * a.v[i] + (1.f - a.b2) * gi * gi;
+  a.m[i] = mi;
+  a.v[i] = vi;
+  const float x = a.w[i] - a.lr * (mi / c1) / (sqrtf(vi / c2) + a.eps);
+  a.w[i] = x;
+  a.Copy(i, x);
 }
 
 __global__ void ZeroFloatKernel(size_t n, float *p) {
@@ -329,9 +619,9 @@ __global__ void ZeroFloatKernel(size_t n, float *p) {
   if (i < n) p[i] = 0.f;
 }
 
-__global__ void ToBf16Kernel(size_t n, const float *src, uint16_t *dst) {
+__global__ void CopyBf16Kernel(size_t n, Adam a) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = F2Bf(src[i]);
+  if (i < n) a.Copy(i, a.w[i]);
 }
 
 inline unsigned Blocks(size_t n, unsigned t = 256) { return (unsigned)((n + t - 1) / t); }
@@ -523,68 +813,81 @@ __global__ void __launch_bounds__(kInferWaves * 64) __attribute__((amdgpu_waves_
   }
 }
 
-// K splits for a weight gradient of `tiles` output tiles and K = batch:
-// about 512 blocks, each with at least four 64-steps of K
-inline int SplitK(int K, int tiles) {
-  const int steps = (K + kGemmK - 1) / kGemmK;
-  return std::max(1, std::min(512 / tiles, steps / 4));
+// Slices of the batch for a weight gradient, each of at least 256 rows; and a
+// slice's rows, in whole K steps.
+inline void SplitBatch(int B, int most, int *slices, int *rows) {
+  most = std::max(1, std::min(most, B / 256));
+  *rows = ((B + most - 1) / most + kGemmK - 1) / kGemmK * kGemmK;
+  *slices = (B + *rows - 1) / *rows;
 }
 
-// split_k > 1 only for kEpiStore into a zeroed C
-template <int EPI>
-void Gemm(hipStream_t s, int M, int N, int K, const uint16_t *A, long sam, long sak,
-          const uint16_t *B, long sbn, long sbk, float *C, int ldc, const float *bias = nullptr,
-          uint16_t *Ch = nullptr, const float *z = nullptr, int split_k = 1) {
-  dim3 grid((N + 63) / 64, (M + 63) / 64, split_k);
-  // every operand here has one unit stride: k or the row
-  if (sak == 1 && sbk == 1)
-    hipLaunchKernelGGL((GemmKernel<EPI, true, true>), grid, dim3(256), 0, s, M, N, K, A, sam,
-                       sak, B, sbn, sbk, C, ldc, bias, Ch, z);
-  else if (sak == 1)
-    hipLaunchKernelGGL((GemmKernel<EPI, true, false>), grid, dim3(256), 0, s, M, N, K, A, sam,
-                       sak, B, sbn, sbk, C, ldc, bias, Ch, z);
-  else if (sbk == 1)
-    hipLaunchKernelGGL((GemmKernel<EPI, false, true>), grid, dim3(256), 0, s, M, N, K, A, sam,
-                       sak, B, sbn, sbk, C, ldc, bias, Ch, z);
-  else
-    hipLaunchKernelGGL((GemmKernel<EPI, false, false>), grid, dim3(256), 0, s, M, N, K, A, sam,
-                       sak, B, sbn, sbk, C, ldc, bias, Ch, z);
+inline BatchSplit SplitOf(size_t B) {
+  BatchSplit s;
+  SplitBatch((int)B, kMostW1Slices, &s.w1_slices, &s.w1_rows);
+  SplitBatch((int)B, kMostW2Slices, &s.w2_slices, &s.w2_rows);
+  return s;
 }
 
 }  // namespace
 
+// One allocation for several arrays, each on a 256-byte boundary.
+class Slab {
+ public:
+  template <typename T>
+  void Add(T **p, size_t count) {
+    parts_.push_back({(void **)p, bytes_});
+    bytes_ += (count * sizeof(T) + 255) / 256 * 256;
+  }
+  size_t bytes() const { return bytes_; }
+  void Place(void *base) const {
+    for (const Part &x : parts_) *x.p = (char *)base + x.at;
+  }
+
+ private:
+  struct Part {
+    void **p;
+    size_t at;
+  };
+  std::vector<Part> parts_;
+  size_t bytes_ = 0;
+};
+
 MlpDevice::MlpDevice() {
   count_ = kFlat;
   hipError_t e = hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking);
-  if (e == hipSuccess) e = gz::Malloc((void **)&master_, kFlat * 4);
-  if (e == hipSuccess) e = gz::Malloc((void **)&grad_, kFlat * 4);
-  if (e == hipSuccess) e = gz::Malloc((void **)&m_, kFlat * 4);
-  if (e == hipSuccess) e = gz::Malloc((void **)&v_, kFlat * 4);
-  if (e == hipSuccess) e = hipMemset(m_, 0, kFlat * 4);
-  if (e == hipSuccess) e = hipMemset(v_, 0, kFlat * 4);
-  if (e == hipSuccess) e = gz::Malloc((void **)&w1h_, (size_t)kCostH1 * kCostIn * 2);
-  if (e == hipSuccess) e = gz::Malloc((void **)&w2h_, (size_t)kCostH2 * kCostH1 * 2);
-  if (e == hipSuccess) e = gz::Malloc((void **)&embh_, (size_t)kCostAlphabet * kCostEmbed * 2);
+  Slab slab;
+  slab.Add(&master_, kFlat);
+  slab.Add(&grad_, kFlat + 1);  // and the loss
+  slab.Add(&m_, kFlat);
+  slab.Add(&v_, kFlat);
+  slab.Add(&w1h_, (size_t)kCostH1 * kCostIn);
+  slab.Add(&w2h_, (size_t)kCostH2 * kCostH1);
+  slab.Add(&embh_, (size_t)kCostAlphabet * kCostEmbed);
+  slab.Add(&operands_, (size_t)2 * kCostH1 * (kCostIn + kCostH2));
+  if (e == hipSuccess) e = gz::Malloc(&weights_, slab.bytes());
+  if (e == hipSuccess) slab.Place(weights_);
   init_status_ = e;
 }
 
 MlpDevice::~MlpDevice() {
-  void *ps[] = {master_, grad_, m_,   v_,    w1h_,  w2h_,  embh_, codes_, x_,
-                z1_,     h1_,   z2_,  h2_,   y_,    t_,    loss_, dz2_,   dz2h_,
-                dz1_,    dz1h_, dh1_, dx_};
-  for (void *p : ps)
-    if (p) (void)gz::Free(p);
+  if (weights_) (void)gz::Free(weights_);
+  if (batch_) (void)gz::Free(batch_);
   if (stream_) (void)hipStreamDestroy(stream_);
 }
 
-void MlpDevice::SyncBf16() {
-  hipLaunchKernelGGL(ToBf16Kernel, dim3(Blocks((size_t)kCostH1 * kCostIn)), dim3(256), 0,
-                     stream_, (size_t)kCostH1 * kCostIn, master_ + kOffW1, w1h_);
-  hipLaunchKernelGGL(ToBf16Kernel, dim3(Blocks((size_t)kCostH2 * kCostH1)), dim3(256), 0,
-                     stream_, (size_t)kCostH2 * kCostH1, master_ + kOffW2, w2h_);
-  hipLaunchKernelGGL(ToBf16Kernel, dim3(1), dim3(256), 0, stream_,
-                     (size_t)kCostAlphabet * kCostEmbed, master_ + kOffEmbed, embh_);
+namespace {
+
+Operands OperandsIn(uint16_t *p) {
+  constexpr size_t kW1 = (size_t)kCostH1 * kCostIn, kW2 = (size_t)kCostH2 * kCostH1;
+  return {p, p + kW1, p + 2 * kW1, p + 2 * kW1 + kW2};
 }
+
+Adam AdamOf(float *w, float *m, float *v, uint16_t *w1h, uint16_t *w2h, uint16_t *embh,
+            uint16_t *operands, float lr) {
+  return {w, m, v, w1h, w2h, embh, OperandsIn(operands), lr, 0.9f, 0.999f, 1e-8f};
+}
+
+}  // namespace
 
 hipError_t MlpDevice::SetWeights(const CostModelWeights &w) {
   if (init_status_ != hipSuccess) return init_status_;
@@ -603,7 +906,8 @@ hipError_t MlpDevice::SetWeights(const CostModelWeights &w) {
   if (e == hipSuccess) e = hipMemsetAsync(v_, 0, kFlat * 4, stream_);
   step_ = 0;
   if (e == hipSuccess) {
-    SyncBf16();
+    hipLaunchKernelGGL(CopyBf16Kernel, dim3(Blocks(kFlat)), dim3(256), 0, stream_, kFlat,
+                       AdamOf(master_, m_, v_, w1h_, w2h_, embh_, operands_, 0.f));
     e = hipGetLastError();
   }
   const hipError_t e2 = hipStreamSynchronize(stream_);
@@ -631,51 +935,26 @@ hipError_t MlpDevice::GetWeights(CostModelWeights *w) {
 hipError_t MlpDevice::Reserve(size_t batch) {
   if (init_status_ != hipSuccess) return init_status_;
   if (batch <= cap_) return hipSuccess;
-  void **ps[] = {(void **)&codes_, (void **)&x_,   (void **)&z1_,  (void **)&h1_,
-                 (void **)&z2_,    (void **)&h2_,  (void **)&y_,   (void **)&t_,
-                 (void **)&loss_,  (void **)&dz2_, (void **)&dz2h_, (void **)&dz1_,
-                 (void **)&dz1h_,  (void **)&dh1_, (void **)&dx_};
-  for (void **p : ps)
-    if (*p) {
-      (void)gz::Free(*p);
-      *p = nullptr;
-    }
-  const size_t B = batch;
-  hipError_t e = hipSuccess;
-  auto al = [&](void **p, size_t bytes) {
-    if (e == hipSuccess) e = gz::Malloc(p, std::max<size_t>(bytes, 64));
-  };
-  al((void **)&codes_, B * kCostResidues);
-  al((void **)&x_, B * kCostIn * 2);
-  al((void **)&z1_, B * kCostH1 * 4);
-  al((void **)&h1_, B * kCostH1 * 2);
-  al((void **)&z2_, B * kCostH2 * 4);
-  al((void **)&h2_, B * kCostH2 * 2);
-  al((void **)&y_, B * 4);
-  al((void **)&t_, B * 4);
-  al((void **)&loss_, 64);
-  al((void **)&dz2_, B * kCostH2 * 4);
-  al((void **)&dz2h_, B * kCostH2 * 2);
-  al((void **)&dz1_, B * kCostH1 * 4);
-  al((void **)&dz1h_, B * kCostH1 * 2);
-  al((void **)&dh1_, B * kCostH1 * 4);
-  al((void **)&dx_, B * kCostIn * 4);
-  if (e == hipSuccess) cap_ = batch;
-  return e;
-}
-
-hipError_t MlpDevice::ForwardDevice(size_t n, size_t B) {
-  (void)n;
-  hipStream_t s = stream_;
-  hipLaunchKernelGGL(EmbedKernel, dim3(Blocks(B * kCostIn)), dim3(256), 0, s, (int)B, codes_,
-                     embh_, x_);
-  Gemm<kEpiBiasGelu>(s, (int)B, kCostH1, kCostIn, x_, kCostIn, 1, w1h_, kCostIn, 1, z1_, kCostH1,
-                     master_ + kOffB1, h1_);
-  Gemm<kEpiBiasGelu>(s, (int)B, kCostH2, kCostH1, h1_, kCostH1, 1, w2h_, kCostH1, 1, z2_,
-                     kCostH2, master_ + kOffB2, h2_);
-  hipLaunchKernelGGL(OutputKernel, dim3(Blocks(B)), dim3(256), 0, s, (int)B, h2_,
-                     master_ + kOffW3, master_ + kOffB3, y_);
-  return hipGetLastError();
+  cap_ = 0;
+  if (batch_) (void)gz::Free(batch_);
+  batch_ = nullptr;
+  Slab slab;
+  slab.Add(&codes_, batch * kCostResidues);
+  slab.Add(&h1_, batch * kCostH1);
+  slab.Add(&t_, batch);
+  slab.Add(&dz2h_, batch * kCostH2);
+  slab.Add(&dz1h_, batch * kCostH1);
+  slab.Add(&w1_parts_, (size_t)kMostW1Slices * kCostH1 * kCostIn);
+  slab.Add(&w2_parts_, (size_t)kMostW2Slices * kCostH2 * kCostH1);
+  slab.Add(&sums_, (size_t)kMostBatchBlocks * kSums);
+  const hipError_t e = gz::Malloc(&batch_, slab.bytes());
+  if (e != hipSuccess) {
+    batch_ = nullptr;
+    return e;
+  }
+  slab.Place(batch_);
+  cap_ = batch;
+  return hipSuccess;
 }
 
 hipError_t MlpDevice::InferDevice(const uint8_t *d_codes, size_t n, float *d_out,
@@ -731,9 +1010,11 @@ hipError_t MlpDevice::TrainStep(const uint8_t *codes, const float *targets, size
   (void)hipMemcpyAsync(codes_, codes, n * kCostResidues, hipMemcpyHostToDevice, s);
   (void)hipMemsetAsync(t_, 0, B * 4, s);
   (void)hipMemcpyAsync(t_, targets, n * 4, hipMemcpyHostToDevice, s);
-  e = StepOnDevice(n, B, lr, 0, nullptr);
+  hipLaunchKernelGGL(ZeroFloatKernel, dim3(1), dim3(64), 0, s, (size_t)1, grad_ + kFlat);
+  if (lr != 0.f) ++step_;
+  e = StepOnDevice(codes_, t_, nullptr, n, B, lr, step_, grad_ + kFlat, true);
   if (e != hipSuccess) return e;
-  if (loss) (void)hipMemcpyAsync(loss, loss_, 4, hipMemcpyDeviceToHost, s);
+  if (loss) (void)hipMemcpyAsync(loss, grad_ + kFlat, 4, hipMemcpyDeviceToHost, s);
   if (flat_grad) (void)hipMemcpyAsync(flat_grad, grad_, kFlat * 4, hipMemcpyDeviceToHost, s);
   return hipStreamSynchronize(s);
 }
@@ -750,60 +1031,33 @@ hipError_t MlpDevice::TrainEpochs(const uint8_t *codes, const float *targets, si
   hipStream_t s = stream_;
   uint8_t *d_codes = nullptr;
   float *d_t = nullptr, *d_sum = nullptr;
-  uint32_t *d_order = nullptr, *d_done = nullptr;
+  uint32_t *d_order = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  e = gz::Malloc((void **)&d_codes, n * kCostResidues);
-  if (e == hipSuccess) e = gz::Malloc((void **)&d_t, n * 4);
-  if (e == hipSuccess) e = gz::Malloc((void **)&d_order, m * 4);
-  if (e == hipSuccess) e = gz::Malloc((void **)&d_sum, 256);
-  d_done = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(d_sum) + 128);
+  Slab slab;
+  slab.Add(&d_codes, n * kCostResidues);
+  slab.Add(&d_t, n);
+  slab.Add(&d_order, m);
+  slab.Add(&d_sum, 1);
+  void *set = nullptr;
+  size_t capacity = 0;
+  e = WorkspacePool::Take(slab.bytes(), &set, &capacity);
+  if (e != hipSuccess) return e;
+  slab.Place(set);
   if (e == hipSuccess) e = hipEventCreate(&e0);
   if (e == hipSuccess) e = hipEventCreate(&e1);
   if (e == hipSuccess)
     e = hipMemcpyAsync(d_codes, codes, n * kCostResidues, hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(d_t, targets, n * 4, hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(d_order, order, m * 4, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipMemsetAsync(d_sum, 0, 256, s);
+  if (e == hipSuccess) e = hipMemsetAsync(d_sum, 0, 4, s);
   if (e == hipSuccess) e = hipEventRecord(e0, s);
   // whole batches only (the remainder of the order is left out, as the
-  // per-step loop of the callers does); every step reads its batch and its
-  // Adam step number from d_done, so a captured run of kGraphSteps steps is
-  // replayed as is
+  // per-step loop of the callers does); the steps' three launches each are
+  // queued ahead of the device
   const size_t steps = m / batch;
-  const long base = step_;
-  auto step = [&]() -> hipError_t {
-    hipLaunchKernelGGL(GatherRowsKernel, dim3((unsigned)Blocks(B * kCostResidues / 16)),
-                       dim3(256), 0, s, d_codes, d_t, d_order, d_done, (int)batch, (int)B,
-                       codes_, t_);
-    hipError_t r = StepOnDevice(batch, B, lr, base, d_done);
-    if (r == hipSuccess) {
-      hipLaunchKernelGGL(AdvanceKernel, dim3(1), dim3(64), 0, s, loss_, d_sum, d_done);
-      r = hipGetLastError();
-    }
-    return r;
-  };
-  constexpr size_t kGraphSteps = 16;
-  size_t done = 0;
-  if (e == hipSuccess && steps >= 2 * kGraphSteps) {
-    {
-      std::lock_guard<std::recursive_mutex> lock(CaptureLock());
-      e = hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed);
-      hipError_t ec = hipSuccess;
-      for (size_t k = 0; k < kGraphSteps && e == hipSuccess; ++k) e = step();
-      ec = hipStreamEndCapture(s, &graph);
-      if (e == hipSuccess) e = ec;
-    }
-    if (e == hipSuccess) e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    // each replay waits for the previous one (one stream); the host
-    // synchronizes between replays so that a replay never races the next
-    for (; e == hipSuccess && done + kGraphSteps <= steps; done += kGraphSteps) {
-      e = hipGraphLaunch(exec, s);
-      if (e == hipSuccess) e = hipStreamSynchronize(s);
-    }
-  }
-  for (; e == hipSuccess && done < steps; ++done) e = step();
+  for (size_t done = 0; e == hipSuccess && done < steps; ++done)
+    e = StepOnDevice(d_codes, d_t, d_order + done * batch, batch, B, lr, step_ + (long)done + 1,
+                     d_sum, false);
   if (e == hipSuccess) e = hipEventRecord(e1, s);
   float sum = 0.f;
   if (e == hipSuccess) e = hipMemcpyAsync(&sum, d_sum, 4, hipMemcpyDeviceToHost, s);
@@ -813,68 +1067,35 @@ hipError_t MlpDevice::TrainEpochs(const uint8_t *codes, const float *targets, si
   float ms = 0.f;
   if (e == hipSuccess && kernel_ms && hipEventElapsedTime(&ms, e0, e1) == hipSuccess)
     *kernel_ms = ms;
-  if (exec) (void)hipGraphExecDestroy(exec);
-  if (graph) (void)hipGraphDestroy(graph);
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
-  for (void *p : {(void *)d_codes, (void *)d_t, (void *)d_order, (void *)d_sum})
-    if (p) (void)gz::Free(p);
+  if (e != hipSuccess) (void)hipStreamSynchronize(s);  // nothing may still read the set
+  WorkspacePool::Give(set, capacity);
   return e;
 }
 
-// One optimisation step on the batch in codes_ / t_ (n rows, B padded):
-// forward, loss, backward, Adam (lr != 0); nothing is read back.  With
-// done, Adam's step number is base + *done + 1 on the device (the host's
-// step count is the caller's to advance); without, the step is counted here.
-hipError_t MlpDevice::StepOnDevice(size_t n, size_t B, float lr, long base,
-                                   const uint32_t *done) {
+// One optimisation step on a batch of n rows (padded to B) of codes and
+// targets, taken through order (may be null); the batch's loss is added to
+// *loss, and with keep the gradient left in grad_.  step: Adam's, from 1.
+// Nothing is read back.
+hipError_t MlpDevice::StepOnDevice(const uint8_t *codes, const float *targets,
+                                   const uint32_t *order, size_t n, size_t B, float lr, long step,
+                                   float *loss, bool keep) {
   hipStream_t s = stream_;
-  hipError_t e = ForwardDevice(n, B);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(LossKernel, dim3(1), dim3(256), 0, s, (int)B, (int)n, y_, t_, y_, loss_);
-  // y_ now holds dY; the gradient is cleared by a kernel (graph-safe)
-  hipLaunchKernelGGL(ZeroFloatKernel, dim3(Blocks(kFlat)), dim3(256), 0, s, kFlat, grad_);
-  const unsigned row_split = std::max(1u, std::min(64u, (unsigned)(B / 64)));
-  // dW3 = H2^T dY, dB3 = sum dY, then dZ2
-  hipLaunchKernelGGL((ColumnSumKernel<uint16_t>), dim3(1, row_split), dim3(256), 0, s, (int)B,
-                     kCostH2, h2_, y_, grad_ + kOffW3);
-  hipLaunchKernelGGL((ColumnSumKernel<float>), dim3(1, row_split), dim3(256), 0, s, (int)B, 1, y_,
-                     (const float *)nullptr, grad_ + kOffB3);
-  hipLaunchKernelGGL(OutputBackwardKernel, dim3(Blocks(B * kCostH2)), dim3(256), 0, s, (int)B,
-                     y_, z2_, master_ + kOffW3, dz2_, dz2h_);
-  // dW2 = dZ2^T H1
-  Gemm<kEpiStore>(s, kCostH2, kCostH1, (int)B, dz2h_, 1, kCostH2, h1_, 1, kCostH1,
-                  grad_ + kOffW2, kCostH1, nullptr, nullptr, nullptr, SplitK((int)B, 4));
-  hipLaunchKernelGGL((ColumnSumKernel<float>), dim3(1, row_split), dim3(256), 0, s, (int)B,
-                     kCostH2, dz2_, (const float *)nullptr, grad_ + kOffB2);
-  // dZ1 = (dZ2 W2) * gelu'(Z1)
-  Gemm<kEpiGeluGrad>(s, (int)B, kCostH1, kCostH2, dz2h_, kCostH2, 1, w2h_, 1, kCostH1, dz1_,
-                     kCostH1, nullptr, dz1h_, z1_);
-  // dW1 = dZ1^T X
-  Gemm<kEpiStore>(s, kCostH1, kCostIn, (int)B, dz1h_, 1, kCostH1, x_, 1, kCostIn,
-                  grad_ + kOffW1, kCostIn, nullptr, nullptr, nullptr, SplitK((int)B, 64));
-  hipLaunchKernelGGL((ColumnSumKernel<float>), dim3(kCostH1 / 64, row_split), dim3(256), 0, s,
-                     (int)B, kCostH1, dz1_, (const float *)nullptr, grad_ + kOffB1);
-  // dX = dZ1 W1, then the embedding gradient
-  Gemm<kEpiStore>(s, (int)B, kCostIn, kCostH1, dz1h_, kCostH1, 1, w1h_, 1, kCostIn, dx_,
-                  kCostIn);
-  hipLaunchKernelGGL(EmbedBackwardKernel, dim3(std::min<size_t>(Blocks(B * kCostIn), 1024)),
-                     dim3(256), 0, s, (int)n, codes_, dx_, grad_ + kOffEmbed);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if (lr != 0.f) {
-    const float b1 = 0.9f, b2 = 0.999f;
-    if (done) {
-      hipLaunchKernelGGL(AdamCountedKernel, dim3(Blocks(kFlat)), dim3(256), 0, s, kFlat,
-                         master_, grad_, m_, v_, lr, b1, b2, 1e-8f, base, done);
-    } else {
-      ++step_;
-      const float c1 = 1.f - std::pow(b1, (float)step_), c2 = 1.f - std::pow(b2, (float)step_);
-      hipLaunchKernelGGL(AdamKernel, dim3(Blocks(kFlat)), dim3(256), 0, s, kFlat, master_,
-                         grad_, m_, v_, lr, b1, b2, c1, c2, 1e-8f);
-    }
-    SyncBf16();
-  }
+  const BatchSplit split = SplitOf(B);
+  const BatchRows rows = {codes, targets, order, (int)n};
+  const int tiles = (int)(B / kRows), batch_blocks = std::min(tiles, kMostBatchBlocks);
+  hipLaunchKernelGGL(BatchKernel, dim3((unsigned)batch_blocks), dim3(256), 0, s, rows, tiles,
+                     embh_, OperandsIn(operands_), master_ + kOffB1, master_ + kOffB2,
+                     master_ + kOffW3, master_ + kOffB3, codes_, h1_, dz2h_, dz1h_, sums_);
+  const unsigned blocks = (unsigned)(kW1Tiles * split.w1_slices + kW2Tiles * split.w2_slices) +
+                          (kSums + 63) / 64;
+  hipLaunchKernelGGL(WeightGradKernel, dim3(blocks), dim3(256), 0, s, (int)B, split, h1_, dz1h_,
+                     dz2h_, codes_, embh_, w1_parts_, w2_parts_, sums_, batch_blocks, grad_, loss);
+  const Adam a = AdamOf(master_, m_, v_, w1h_, w2h_, embh_, operands_, lr);
+  const float c1 = 1.f - std::pow(a.b1, (float)step), c2 = 1.f - std::pow(a.b2, (float)step);
+  hipLaunchKernelGGL(AdamKernel, dim3(Blocks(kFlat)), dim3(256), 0, s, kFlat, a, grad_, split,
+                     w1_parts_, w2_parts_, c1, c2, keep ? 1 : 0);
   return hipGetLastError();
 }
 
