@@ -1038,8 +1038,8 @@ __global__ void __launch_bounds__(kWave)
 // job is its query side (frames of reads: up to 50 residues from a seed
 // anywhere in them).  Calls that bring no order of their own get one, longest
 // sides first, in two passes over the positions: 1,000,003 extensions of reads
-// 1.23 -> 0.89 ms, 0.03 of that for the order (by the extensions' true cell
-// counts it would be 0.86).  Lengths from kSideBins - 1 on are one bin.
+// 1.23 -> 0.89 ms, 0.04 of that for the order (by the extensions' true cell
+// counts it would be 0.87).  Lengths from kSideBins - 1 on are one bin.
 constexpr uint32_t kSideBins = 64;
 constexpr uint32_t kSideItems = 16;
 constexpr uint32_t kSideChunk = 256 * kSideItems;  // jobs per block
@@ -1484,6 +1484,15 @@ inline uint32_t WideSlotsFor(uint32_t wide) {
 enum : int { kWaveAuto = 0, kWaveNever = 1, kWaveDirect = 2 };
 constexpr uint32_t kRunCounters = 8 + 2 * kSideBins;
 
+// Jobs up to which a call runs one wave per job (wave_dp.h), by the longest
+// query that the handle is told.  Frames of reads (a 64-column ring): a wave
+// per job takes 4.0 ns a job, a lane per job 0.28 ms however few they are, the
+// time of one long extension on a lane.  Proteins of 100-500 residues: 11 ns a
+// job (131,072: 1.4 ms), and 2.6 ms on lanes; the line for longer queries lies
+// lower than theirs, since translated reads are told as all their frames.
+constexpr size_t kRowJobsShort = 65536, kRowJobsLong = 131072;
+inline size_t RowJobsFor(uint32_t wide) { return wide <= 64 ? kRowJobsShort : kRowJobsLong; }
+
 struct gz_gapped_extender_s {
   uint32_t delimiter = kDelimiter;
   const uint64_t *queries = nullptr;
@@ -1501,8 +1510,7 @@ struct gz_gapped_extender_s {
   // workspace
   // [0] jobs out of the narrow ring, [1] failures, [2] jobs of the row
   // kernel past 64 columns, [3] the work queue's head, [4] jobs of the second
-  // overflow list, [5] the row kernel's queue head over the first, [8] on:
-  // jobs per side length bin and the bins' cursors
+  // overflow list, [8] on: jobs per side length bin and the bins' cursors
   uint32_t *counters = nullptr;
   uint32_t *overflow_list = nullptr;   // out of the narrow ring
   uint32_t *overflow_list2 = nullptr;  // for the global ring
@@ -1606,16 +1614,13 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
   const WaveDpParams R = {P.queries, P.database, P.delim, P.gap_open + P.gap_ext,
                           P.gap_ext, P.cutoff, kWaveDpMargin};
   const uint32_t *none = nullptr;
-#define GZ_ROWS(N, LIST, COUNT, ORDER, HEAD, NARROW)                                            \
-  {                                                                                             \
-    const WaveDpGrid g = WaveDpGridFor(N);                                                      \
-    hipLaunchKernelGGL((GappedRowKernel<kReverse>), dim3(g.blocks), dim3(kWaveDpBlock), 0, s,    \
-                       (uint32_t)(N), LIST, COUNT, ORDER, (uint32_t)size, g.batch, HEAD, R,      \
-                       h->matrix, h->number_letters, d_q, d_d, d_scores, d_cells, list2_out,     \
-                       w.overflow_list2, (int)h->narrow, NARROW, wide_out, failures);            \
-  }
-  const bool row_jobs = rows && size <= kWaveDpJobs;
-  if (!order && wide_first == 0 && size > kWaveDpJobs) {
+#define GZ_ROWS(N, LIST, COUNT, ORDER, NARROW)                                                  \
+  hipLaunchKernelGGL((GappedRowKernel<kReverse>), dim3(WaveDpBlocksFor(N)), dim3(kWaveDpBlock), \
+                     0, s, (uint32_t)(N), LIST, COUNT, ORDER, (uint32_t)size, R, h->matrix,     \
+                     h->number_letters, d_q, d_d, d_scores, d_cells, list2_out,                 \
+                     w.overflow_list2, (int)h->narrow, NARROW, wide_out, failures)
+  const bool row_jobs = rows && size <= RowJobsFor(h->wide);
+  if (!order && wide_first == 0 && !row_jobs && size > kRowJobsShort) {
     // the keys and the order lie in the overflow lists: the first ring reads
     // the order and writes the first list, whose keys are read by then; the
     // second list is written after the first ring
@@ -1628,7 +1633,7 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
                        counts + kSideBins, w.overflow_list2);
     order = w.overflow_list2;
   }
-  if (row_jobs) GZ_ROWS(size, none, none, order, w.counters + 3, narrow_out)
+  if (row_jobs) GZ_ROWS(size, none, none, order, narrow_out);
   // 16-bit cells in the LDS rings when the cutoff and gap costs allow them
   // (LaneRingLds16); bands whose scores grow past them move on like bands
   // that outgrow the ring
@@ -1704,7 +1709,7 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
     // count); 16-bit cells leave LDS for more blocks
     if (rows)
       GZ_ROWS(std::min<size_t>(size, kWaveDpJobs), w.overflow_list, narrow_out, none,
-              w.counters + 5, (uint32_t *)nullptr)
+              (uint32_t *)nullptr);
     if (short_cells) GZ_RING64(true, dim3(256u * 6), 0, 0, w.overflow_list, narrow_out, none);
     else GZ_RING64(false, dim3(256u * 4), 0, 0, w.overflow_list, narrow_out, none);
   }
@@ -1767,7 +1772,7 @@ static gz_status GappedReserve(gz_gapped_extender_t h, size_t size, hipStream_t 
   // lanes: one per job at most, at least kWideSlots, within the budget; a
   // call that runs on the row kernel leaves the global ring next to nothing
   // (bands past 128 columns)
-  const bool rows = h->wave_mode == kWaveAuto && size <= kWaveDpJobs &&
+  const bool rows = h->wave_mode == kWaveAuto && size <= RowJobsFor(h->wide) &&
                     WaveDpServes(h->cutoff, h->gap_open, h->gap_ext);
   const size_t by_jobs = rows ? 0 : (size + 63) / 64 * 64;
   const uint32_t want = (uint32_t)std::max<size_t>(

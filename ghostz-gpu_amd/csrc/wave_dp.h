@@ -504,96 +504,109 @@ struct NoOps {
 
 constexpr int kWaveDpBlock = 256;
 
-// Jobs up to which a call runs one wave per job: beyond, the lanes of
-// GappedKernel fill the chip (extensions of reads, one side of 50 residues:
-// 3.0 ns per job here whatever their number; one lane per job takes 170 us
-// however few they are and 1.2 ns per job past 200,000).
+// Jobs out of the first ring up to which they run one wave per job: beyond,
+// the 64-column ring's lanes fill the chip.
 constexpr uint32_t kWaveDpJobs = 1u << 16;
 constexpr uint32_t kWaveDpWaves = 8192;  // resident at once: 8 per SIMD
 
+// The jobs of a block of the one-wave-per-job form: block b of B has jobs b,
+// b + B, b + 2 B, ... (an order by length spreads evenly), which its waves
+// take one by one from a counter in LDS.  Blocks that end early leave their
+// issue slots to the others of the CU.  A counter in memory that all waves
+// share costs 12 ns a request, and every wave makes at least the one that finds
+// no job: 10,000 read extensions took 135 us with it and take 58 so, 45,000
+// 539 and 180; with a quarter of the jobs left to such a counter 135 and 197.
+struct BlockJobs {
+  uint32_t *next;  // in LDS
+  uint32_t k;
+  // by every thread, before the block's next barrier
+  __device__ __forceinline__ void Begin(uint32_t *lds_next) {
+    next = lds_next;
+    k = Uniform(threadIdx.x / kWave);
+    if (threadIdx.x == 0) *next = blockDim.x / kWave;
+  }
+  // the wave's job, or one past the jobs
+  __device__ __forceinline__ uint64_t Job(uint32_t block, uint32_t blocks) const {
+    return (uint64_t)block + (uint64_t)k * blocks;
+  }
+  __device__ __forceinline__ void Advance() {
+    uint32_t v = 0;
+    if (__lane_id() == 0) v = atomicAdd(next, 1u);
+    k = Uniform(v);
+  }
+};
+
 // One wave per job: jobs k (order[k] when `order` is set), or the
 // *list_count jobs of `list` when that is set and they are at most
-// kWaveDpJobs.  A wave takes `batch` slots at a time, its first without
-// asking, the others from *head (zero at the launch).  A job whose band
-// outgrows 128 columns is appended to overflow_list; narrow_count and
-// wide_count (either may be null) count those past narrow_columns and past
-// 64 columns.
+// kWaveDpJobs.  A job whose band outgrows 128 columns is appended to
+// overflow_list; narrow_count and wide_count (either may be null) count those
+// past narrow_columns and past 64 columns.
 template <bool kReverse>
 __global__ void __launch_bounds__(kWaveDpBlock)
     GappedRowKernel(uint32_t n, const uint32_t *list, const uint32_t *list_count,
-                    const uint32_t *order, uint32_t limit, uint32_t batch, uint32_t *head,
-                    WaveDpParams P, const int *matrix, uint32_t nl, uint32_t *qpos,
-                    uint32_t *dpos, int *scores, uint32_t *cells, uint32_t *overflow_count,
-                    uint32_t *overflow_list, int narrow_columns, uint32_t *narrow_count,
-                    uint32_t *wide_count, uint32_t *failed) {
+                    const uint32_t *order, uint32_t limit, WaveDpParams P, const int *matrix,
+                    uint32_t nl, uint32_t *qpos, uint32_t *dpos, int *scores, uint32_t *cells,
+                    uint32_t *overflow_count, uint32_t *overflow_list, int narrow_columns,
+                    uint32_t *narrow_count, uint32_t *wide_count, uint32_t *failed) {
   __shared__ int8_t sm[kTableDim * kScoreStride];
+  __shared__ uint32_t next, counts[2];
   if (list) {
     n = Uniform(*list_count);
     if (n > kWaveDpJobs) return;
   }
-  const uint32_t waves = gridDim.x * (kWaveDpBlock / kWave);
-  const uint32_t wave = blockIdx.x * (kWaveDpBlock / kWave) + Uniform(threadIdx.x / kWave);
-  if (blockIdx.x * (kWaveDpBlock / kWave) * batch >= n) return;  // no job for the block
+  if (blockIdx.x >= n) return;  // no job for the block
+  BlockJobs jobs;
+  jobs.Begin(&next);
+  if (threadIdx.x < 2) counts[threadIdx.x] = 0;
   StageWaveDpScores(sm, matrix, nl);
   __syncthreads();
   const int inc = kReverse ? -1 : 1;
   const bool leads = __lane_id() == 0;
-  for (uint32_t next = wave * batch; next < n;) {
-    const uint32_t stop = next + batch < n ? next + batch : n;
-    for (uint32_t k = next; k < stop; ++k) {
-      const uint32_t i = Uniform(list ? list[k] : order ? order[k] : k);
-      if (i >= limit) {  // an order entry out of range: counted, never read
-        if (leads) atomicAdd(failed, 1u);
-        continue;
-      }
-      const uint32_t q = Uniform(qpos[i]), d = Uniform(dpos[i]);
-      WaveDpBand B;
-      WaveDp<kReverse, 1> x;
-      NoOps none;
-      int r = x.Begin(P, B, q, d);
-      if (r == 0) r = x.Rows(P, sm, B, none);
-      if (r == kWaveDpWiden) {
-        // two columns per lane from here on
-        WaveDp<kReverse, 2> y;
-        y.Widen(P, B, x);
-        r = y.Rows(P, sm, B, none);
-      }
-      if (leads) {
-        if (r == kWaveDpDone) {
-          scores[i] = B.best;
-          qpos[i] = (uint32_t)((int)q + (B.best_col - 1) * inc);
-          dpos[i] = (uint32_t)((int)d + B.best_row * inc);
-          if (cells) cells[i] = (uint32_t)B.cells;
-        } else {
-          overflow_list[atomicAdd(overflow_count, 1u)] = i;
-        }
-        const bool done = r == kWaveDpDone;
-        if (narrow_count && (!done || B.widest > narrow_columns)) atomicAdd(narrow_count, 1u);
-        if (wide_count && (!done || B.widest > 64)) atomicAdd(wide_count, 1u);
-      }
+  for (uint64_t k; (k = jobs.Job(blockIdx.x, gridDim.x)) < n; jobs.Advance()) {
+    const uint32_t i = Uniform(list ? list[k] : order ? order[k] : (uint32_t)k);
+    if (i >= limit) {  // an order entry out of range: counted, never read
+      if (leads) atomicAdd(failed, 1u);
+      continue;
     }
-    if ((uint64_t)waves * batch >= n) break;  // no slots past the first ones
-    uint32_t b = 0;
-    if (leads) b = atomicAdd(head, batch);
-    // below 2^32: the host bounds n and the grid
-    next = waves * batch + Uniform(b);
+    const uint32_t q = Uniform(qpos[i]), d = Uniform(dpos[i]);
+    WaveDpBand B;
+    WaveDp<kReverse, 1> x;
+    NoOps none;
+    int r = x.Begin(P, B, q, d);
+    if (r == 0) r = x.Rows(P, sm, B, none);
+    if (r == kWaveDpWiden) {
+      // two columns per lane from here on
+      WaveDp<kReverse, 2> y;
+      y.Widen(P, B, x);
+      r = y.Rows(P, sm, B, none);
+    }
+    if (leads) {
+      const bool done = r == kWaveDpDone;
+      if (done) {
+        scores[i] = B.best;
+        qpos[i] = (uint32_t)((int)q + (B.best_col - 1) * inc);
+        dpos[i] = (uint32_t)((int)d + B.best_row * inc);
+        if (cells) cells[i] = (uint32_t)B.cells;
+      } else {
+        overflow_list[atomicAdd(overflow_count, 1u)] = i;
+      }
+      if (!done || B.widest > narrow_columns) atomicAdd(&counts[0], 1u);
+      if (!done || B.widest > 64) atomicAdd(&counts[1], 1u);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (narrow_count && counts[0]) atomicAdd(narrow_count, counts[0]);
+    if (wide_count && counts[1]) atomicAdd(wide_count, counts[1]);
   }
 }
 
-// Grid and slots per request of a GappedRowKernel launch over at most `jobs`
-// jobs: as many waves as jobs up to the resident ones, and about eight
-// requests per wave.
-struct WaveDpGrid {
-  uint32_t blocks, batch;
-};
-inline WaveDpGrid WaveDpGridFor(size_t jobs) {
+// Blocks of a GappedRowKernel launch over at most `jobs` jobs: as many waves
+// as jobs up to the resident ones.
+inline uint32_t WaveDpBlocksFor(size_t jobs) {
   const size_t per = kWaveDpBlock / kWave;
   const size_t waves = jobs < kWaveDpWaves ? (jobs > 0 ? jobs : 1) : (size_t)kWaveDpWaves;
-  WaveDpGrid g;
-  g.blocks = (uint32_t)((waves + per - 1) / per);
-  const size_t b = jobs / (g.blocks * per * 8) + 1;
-  g.batch = (uint32_t)(b > 16 ? 16 : b);
-  return g;
+  return (uint32_t)((waves + per - 1) / per);
 }
 
 }  // namespace gz
