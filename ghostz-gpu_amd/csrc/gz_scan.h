@@ -3,8 +3,10 @@
 // and src/device_seeds_memory.cu:28-34).
 //
 // Reduce-then-scan over tiles of 1024 items (256 threads x 4), recursing on
-// the tile aggregates.  Unsigned element types only (identity 0 for both
-// sum and max).
+// the tile aggregates; up to 16,384 items in one block of 1024 threads, since
+// a launch costs more there than the items (2,304 items: three launches of
+// 3 us and the gaps between them, one of 5 us).  Unsigned element types only
+// (identity 0 for both sum and max).
 #pragma once
 
 #include "gz_device.h"
@@ -64,6 +66,36 @@ __global__ void __launch_bounds__(kScanThreads)
   }
 }
 
+// The whole scan in one block of kSmallScanThreads threads, kSmallScanItems
+// consecutive items each.  Safe in place.
+constexpr int kSmallScanThreads = 1024;
+constexpr int kSmallScanItems = 16;
+constexpr size_t kSmallScan = (size_t)kSmallScanThreads * kSmallScanItems;
+
+template <typename T, bool kMax, bool kInclusive>
+__global__ void __launch_bounds__(kSmallScanThreads)
+    ScanSmallKernel(const T *in, T *out, uint32_t n) {
+  __shared__ T lds[kSmallScanThreads / kWave];
+  // as few items per thread as hold n
+  const uint32_t per = (n + kSmallScanThreads - 1) / kSmallScanThreads;
+  const uint32_t base = threadIdx.x * per;
+  T v[kSmallScanItems];
+  T run = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < (uint32_t)kSmallScanItems; ++j) {
+    v[j] = (j < per && base + j < n) ? in[base + j] : T(0);
+    run = kMax ? (v[j] > run ? v[j] : run) : run + v[j];
+  }
+  T inc, acc;
+  BlockScan<T, kMax>(run, lds, &inc, &acc, nullptr);
+#pragma unroll
+  for (uint32_t j = 0; j < (uint32_t)kSmallScanItems; ++j) {
+    const T before = acc;
+    acc = kMax ? (v[j] > acc ? v[j] : acc) : acc + v[j];
+    if (j < per && base + j < n) out[base + j] = kInclusive ? acc : before;
+  }
+}
+
 inline size_t AlignUp(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 template <typename T>
@@ -81,6 +113,15 @@ template <typename T, bool kMax>
 inline hipError_t DeviceScan(const T *in, T *out, size_t n, bool inclusive,
                              void *temp, hipStream_t stream) {
   if (n == 0) return hipSuccess;
+  if (n <= kSmallScan) {
+    if (inclusive)
+      hipLaunchKernelGGL((ScanSmallKernel<T, kMax, true>), dim3(1), dim3(kSmallScanThreads), 0,
+                         stream, in, out, (uint32_t)n);
+    else
+      hipLaunchKernelGGL((ScanSmallKernel<T, kMax, false>), dim3(1), dim3(kSmallScanThreads), 0,
+                         stream, in, out, (uint32_t)n);
+    return hipGetLastError();
+  }
   const size_t tiles = (n + kScanTile - 1) / kScanTile;
   T *agg = nullptr;
   if (tiles > 1) {

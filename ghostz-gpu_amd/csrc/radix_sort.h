@@ -1,8 +1,8 @@
 // radix_sort.h -- stable device sort of (u32 key, u32 value) pairs, the
 // project's own replacement for a library radix sort.
 //
-// LSD passes of 8 bits.  A pass: per-tile digit histograms (tiles of 4096
-// items, digit-major so that one exclusive scan gives every (digit, tile)
+// LSD passes of 8 bits.  A pass: per-tile digit histograms (tiles of 1024 to
+// 4096 items, digit-major so that one exclusive scan gives every (digit, tile)
 // its output offset), then a scatter in which each wave ranks its 64 items
 // among equal digits with eight ballots, and the waves' counts are
 // prefix-summed in LDS in item order, so equal keys keep their input order.

@@ -10,18 +10,26 @@ namespace gz {
 namespace {
 
 constexpr int kSortThreads = 256;
-constexpr int kSortItems = 16;                          // per thread
-constexpr size_t kSortTile = kSortThreads * kSortItems;  // 4096
-constexpr int kSubChunks = kSortTile / kWave;            // 64 runs of 64 items
 constexpr int kDigits = 256;
 
+// Items per thread: a tile's ranking is a serial chain over its runs of 64
+// items (17 us for a tile of 4096), so sorts that leave the chip idle take
+// smaller tiles, as long as one block scans their histograms (gz_scan.h).
+// 34,586 pairs over 32 bits: 130 us in tiles of 4096, 60 us in tiles of 1024.
+inline int SortItems(size_t n) { return n <= 65536 ? 4 : n <= 131072 ? 8 : 16; }
+inline size_t SortTiles(size_t n) {
+  const size_t tile = (size_t)kSortThreads * SortItems(n);
+  return (n + tile - 1) / tile;
+}
+
+template <int kSortItems>
 __global__ void __launch_bounds__(kSortThreads)
     DigitHistogramKernel(const uint32_t *keys, size_t n, int shift, uint32_t tiles,
                          uint32_t *hist) {
   __shared__ uint32_t count[kDigits];
   count[threadIdx.x] = 0;
   __syncthreads();
-  const size_t base = (size_t)blockIdx.x * kSortTile;
+  const size_t base = (size_t)blockIdx.x * (kSortThreads * kSortItems);
 #pragma unroll 4
   for (int j = 0; j < kSortItems; ++j) {
     const size_t i = base + (size_t)j * kSortThreads + threadIdx.x;
@@ -32,17 +40,19 @@ __global__ void __launch_bounds__(kSortThreads)
 }
 
 // Item s * 64 + lane of the tile is handled by wave s % 4 as its item s / 4.
+template <int kSortItems>
 __global__ void __launch_bounds__(kSortThreads)
     DigitScatterKernel(const uint32_t *keys, const uint32_t *values, size_t n, int shift,
                        uint32_t tiles, const uint32_t *offsets, uint32_t *keys_out,
                        uint32_t *values_out) {
-  __shared__ uint16_t count[kSubChunks][kDigits];  // 32 KB
+  constexpr int kSubChunks = kSortThreads * kSortItems / kWave;  // runs of 64 items
+  __shared__ uint16_t count[kSubChunks][kDigits];  // up to 32 KB
   for (int i = threadIdx.x; i < kSubChunks * kDigits; i += kSortThreads)
     (&count[0][0])[i] = 0;
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  const size_t base = (size_t)blockIdx.x * kSortTile;
+  const size_t base = (size_t)blockIdx.x * (kSortThreads * kSortItems);
   uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
 #pragma unroll
   for (int j = 0; j < kSortItems; ++j) {
@@ -89,7 +99,7 @@ __global__ void __launch_bounds__(kSortThreads)
 }  // namespace
 
 size_t RadixSortTempBytes(size_t n) {
-  const size_t tiles = (n + kSortTile - 1) / kSortTile;
+  const size_t tiles = SortTiles(n);
   const size_t h = AlignUp(tiles * kDigits * sizeof(uint32_t), 256);
   return 2 * h + DeviceScanTempBytes<uint32_t>(tiles * kDigits);
 }
@@ -99,21 +109,28 @@ hipError_t RadixSortPairs(uint32_t *keys, uint32_t *values, uint32_t *keys_alt,
                           hipStream_t s) {
   if (n == 0) return hipSuccess;
   if (bits <= 0 || bits > 32 || bits % 16 != 0 || n > 0xffffffffull) return hipErrorInvalidValue;
-  const size_t tiles = (n + kSortTile - 1) / kSortTile;
+  const size_t tiles = SortTiles(n);
   const size_t h = AlignUp(tiles * kDigits * sizeof(uint32_t), 256);
   uint32_t *hist = (uint32_t *)temp;
   uint32_t *offs = (uint32_t *)((char *)temp + h);
   void *scan_tmp = (char *)temp + 2 * h;
   uint32_t *src_k = keys, *src_v = values, *dst_k = keys_alt, *dst_v = values_alt;
   for (int shift = 0; shift < bits; shift += 8) {
-    hipLaunchKernelGGL(DigitHistogramKernel, dim3((unsigned)tiles), dim3(kSortThreads), 0, s,
-                       src_k, n, shift, (uint32_t)tiles, hist);
+    const int items = SortItems(n);
+    hipLaunchKernelGGL(items == 4   ? DigitHistogramKernel<4>
+                       : items == 8 ? DigitHistogramKernel<8>
+                                    : DigitHistogramKernel<16>,
+                       dim3((unsigned)tiles), dim3(kSortThreads), 0, s, src_k, n, shift,
+                       (uint32_t)tiles, hist);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
       e = DeviceScan<uint32_t, false>(hist, offs, tiles * kDigits, false, scan_tmp, s);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(DigitScatterKernel, dim3((unsigned)tiles), dim3(kSortThreads), 0, s,
-                       src_k, src_v, n, shift, (uint32_t)tiles, offs, dst_k, dst_v);
+    hipLaunchKernelGGL(items == 4   ? DigitScatterKernel<4>
+                       : items == 8 ? DigitScatterKernel<8>
+                                    : DigitScatterKernel<16>,
+                       dim3((unsigned)tiles), dim3(kSortThreads), 0, s, src_k, src_v, n, shift,
+                       (uint32_t)tiles, offs, dst_k, dst_v);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     uint32_t *t = src_k;
