@@ -158,7 +158,7 @@ class Aligner : public PresearchDevice {
   hipEvent_t run_ev_[2][2] = {};  // per slot: around its gapped kernels
   std::mutex stats_mutex_;        // AlignStats updates from both slots
   TracebackRunner tracebacks_;    // the result build's
-  uint32_t max_query_length_ = 0;
+  uint32_t max_query_length_ = 0, longest_side_ = 0;
   // pinned job buffers per pipeline slot
   std::vector<std::pair<void *, size_t> > pinned_jobs_;
   // the learned schedule's gate (query side residues)

@@ -175,6 +175,11 @@ int Aligner::BeginQueryChunk(const QuerySet &q, const std::vector<uint8_t> &conc
     byte_tables = byte_tables && v >= -127 && v <= 127;
   }
   max_query_length_ = q.max_length;
+  longest_side_ = q.max_length;
+  if (q.translated) {  // a frame
+    longest_side_ = 0;
+    for (uint32_t l : q.dna_lengths) longest_side_ = std::max(longest_side_, l / 3);
+  }
   hipStream_t s = stream_;
   uint64_t *d_q = nullptr;
   int *d_cut = nullptr, *d_trig = nullptr;
@@ -580,9 +585,10 @@ int Aligner::Tracebacks(size_t ci, const std::vector<TracebackJob> &jobs, int cu
   const size_t n = jobs.size();
   out->resize(n);
   if (n == 0) return 0;
-  const TracebackInputs in = {dq_.packed,        chunks_[ci]->packed,   max_query_length_,
-                              db_->max_length,   d_matrix_,             opt_.search.nl,
-                              opt_.search.gap_open, opt_.search.gap_extension, cutoff};
+  const TracebackInputs in = {dq_.packed,      chunks_[ci]->packed,  max_query_length_,
+                              db_->max_length, longest_side_,        d_matrix_,
+                              opt_.search.nl,  opt_.search.gap_open, opt_.search.gap_extension,
+                              cutoff};
   float ms = 0;
   GZ_TRY(tracebacks_.Run(in, jobs.data(), (uint32_t)n, out->data(), traceback_stream_, &ms));
   st->traceback_kernel_ms += ms;

@@ -462,8 +462,9 @@ gz_status gz_build_results(const uint64_t *pq, const uint64_t *pd, const gz_trac
   GZ_REQUIRE(n < (1ull << 31), "gz_build_results: too many jobs");
   if (n == 0) return GZ_OK;
   hipStream_t s = stream ? stream->s : nullptr;
-  const TracebackInputs in = {pq,       pd,      max_query_length, max_subject_length, d_matrix, nl,
-                              gap_open, gap_ext, cutoff};
+  const TracebackInputs in = {pq,       pd,       max_query_length, max_subject_length,
+                              max_query_length, d_matrix, nl,       gap_open,
+                              gap_ext,  cutoff};
   TracebackRunner run(/*pooled=*/true);
   const hipError_t e = run.Run(in, reinterpret_cast<const TracebackJob *>(jobs), (uint32_t)n,
                                reinterpret_cast<TracebackOut *>(results), s, nullptr);

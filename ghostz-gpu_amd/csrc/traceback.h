@@ -23,6 +23,7 @@ constexpr uint32_t kTracebackArena = 1u << 16;
 struct TracebackInputs {
   const uint64_t *queries, *database;
   uint32_t max_query_length, max_subject_length;
+  uint32_t longest_side;  // residues between two of a query's delimiters, at most
   const int *matrix;  // on the device
   uint32_t nl;
   int gap_open, gap_ext, cutoff;

@@ -419,6 +419,11 @@ struct TracebackHalf {
 constexpr uint32_t kNeedsLane = 4;
 
 constexpr int kTbWaveBlock = 256;
+// Results of one call from which sides that fit the lanes' LDS columns take a
+// lane each again, where the lanes' scratch (11 GB) is kept: on read results a
+// call takes 24 ns each on waves, and 1.4 ms and 13 ns each on lanes (843,199
+// in one call: 20.3 ms on waves, 12.5 on lanes).
+constexpr uint32_t kLaneResults = 131072;
 // Waves resident at once: four per SIMD, enough to hide a row's dependent
 // steps behind the other waves' instructions.
 constexpr uint32_t kTbWaves = 4096;
@@ -815,7 +820,8 @@ hipError_t TracebackRunner::Queue(const TracebackInputs &in, const TracebackJob 
       if (c != hipSuccess) return c;
     }
   // the wave form's rows of the longest subject must fit 32-bit offsets
-  const bool waves = WaveDpServes(in.cutoff, in.gap_open, in.gap_ext) &&
+  const bool many_short = !pooled_ && n > kLaneResults && in.longest_side + 2 <= kTbLdsCols;
+  const bool waves = !many_short && WaveDpServes(in.cutoff, in.gap_open, in.gap_ext) &&
                      in.max_subject_length < (1u << 27) && in.max_query_length < (1u << 27);
   const uint32_t per = kTbWaveBlock / kWave;
   WaveCaps wc = {};

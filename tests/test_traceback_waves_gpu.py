@@ -170,3 +170,17 @@ def test_concurrent_calls():
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_many_short_results_take_lanes():
+    """One call of more than 131,072 read results runs a lane each in an
+    aligner; the batched form's blocks of the same search run on waves.  The
+    outputs are byte-identical."""
+    import synthetic
+    q, d = synthetic.translated_workload(8, 20000, 24000)
+    queries, database = gz.Queries(*q, translated=True), gz.Database(*d)
+    print("traceback: one large call and its blocks", flush=True)
+    one, st = gz.Aligner(database).align(queries)
+    blocks, _ = gz.Aligner(database, batched=1).align(queries)
+    assert st["results"] > 131072
+    assert one == blocks
