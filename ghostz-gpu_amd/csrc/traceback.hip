@@ -437,7 +437,12 @@ struct WaveCaps {
 // Records the operations of WaveDp's rows in the reference's layout.  A row's
 // cells past its new band end are overwritten by the following rows or never
 // read but as unwritten, so a row stores the columns [start, new end) only
-// and every byte has one writer.
+// and every byte has one writer.  The horizontal gap lacks the reference's
+// reset after a pruned cell, so kExt1 of a kept cell may be set where the
+// reference's is not.  No path reads it there: a path comes to a cell in a
+// horizontal gap only from the cell's right neighbour in the same row, and the
+// gap into that neighbour is at least the running best less the cutoff, which
+// a gap through a pruned cell is below.
 struct ArenaOps {
   uint8_t *arena;
   int2 *rows;  // (base, off)

@@ -12,11 +12,13 @@
 // form for calls with too few jobs to fill the chip with a lane each, and
 // for bands that outgrow the lanes' first LDS ring.  Measured per call
 // against the lane forms: 300 read extensions 310 -> 25 us, 20,011 of
-// proteins of 100-500 residues 4.0 -> 0.39 ms, 3,001 of Pareto lengths up to
-// 35,000 99.8 -> 11 ms; 1,000,003 of reads (first ring on lanes, its
+// proteins of 100-500 residues 4.0 -> 0.31 ms, 3,001 of Pareto lengths up to
+// 35,000 99.8 -> 10 ms; 1,000,003 of reads (first ring on lanes, its
 // overflow here) 1.38 -> 1.24 ms.  C is 1 and widens to 2 when a band needs
 // it: with one column per lane nothing inside a lane is serial, and bands
-// at the presearch's cutoff are 15 to 30 columns wide.
+// at the presearch's cutoff are 15 to 30 columns wide.  The result build
+// (traceback.hip) records the operations of the same rows, in windows of up
+// to 4 columns per lane at its higher cutoff.
 //
 // The row recurrence is GappedOneSide's (src/gapped_extender.cpp:306-471),
 // with the two values that it carries from column to column as scans:
