@@ -1042,7 +1042,7 @@ __global__ void __launch_bounds__(kWave)
 // counts it would be 0.87).  Lengths from kSideBins - 1 on are one bin.
 constexpr uint32_t kSideBins = 64;
 constexpr uint32_t kSideItems = 16;
-constexpr uint32_t kSideChunk = 256 * kSideItems;  // jobs per block
+constexpr uint32_t kSideChunk = 256 * kSideItems;  // jobs of a block at a time
 
 // Fields of a packed word equal to `code`, as their high bits.
 __device__ __forceinline__ uint64_t FieldsEqual(uint64_t word, uint32_t code) {
@@ -1095,14 +1095,17 @@ __global__ void __launch_bounds__(256)
   __shared__ uint32_t hist[kSideBins];
   if (threadIdx.x < kSideBins) hist[threadIdx.x] = 0;
   __syncthreads();
-  const uint32_t begin = blockIdx.x * kSideChunk + threadIdx.x;
+  for (size_t chunk = (size_t)blockIdx.x * kSideChunk; chunk < n;
+       chunk += (size_t)gridDim.x * kSideChunk) {
+    const uint32_t begin = (uint32_t)chunk + threadIdx.x;
 #pragma unroll 4
-  for (uint32_t r = 0; r < kSideItems; ++r) {
-    const uint32_t i = begin + r * 256;
-    if (i >= n) break;
-    const uint32_t key = SideLength<kReverse>(queries, qpos[i], delim);
-    keys[i] = (uint8_t)key;
-    atomicAdd(&hist[key], 1u);
+    for (uint32_t r = 0; r < kSideItems; ++r) {
+      const uint32_t i = begin + r * 256;
+      if (i >= n) break;
+      const uint32_t key = SideLength<kReverse>(queries, qpos[i], delim);
+      keys[i] = (uint8_t)key;
+      atomicAdd(&hist[key], 1u);
+    }
   }
   __syncthreads();
   if (threadIdx.x < kSideBins && hist[threadIdx.x])
@@ -1116,30 +1119,34 @@ __global__ void __launch_bounds__(256)
                     uint32_t *order) {
   __shared__ uint32_t next[kSideBins];
   static_assert(kSideBins == kWave, "a lane per bin");
-  if (threadIdx.x < kSideBins) next[threadIdx.x] = 0;
-  __syncthreads();
-  const uint32_t begin = blockIdx.x * kSideChunk + threadIdx.x;
-  uint32_t key[kSideItems];
+  // the jobs of the bins above a lane's, lane l having bin kSideBins - 1 - l
+  const uint32_t bin = kSideBins - 1 - threadIdx.x % kSideBins;
+  const uint32_t count = counts[bin], before = WaveInclusiveSum(count) - count;
+  for (size_t chunk = (size_t)blockIdx.x * kSideChunk; chunk < n;
+       chunk += (size_t)gridDim.x * kSideChunk) {
+    if (threadIdx.x < kSideBins) next[threadIdx.x] = 0;
+    __syncthreads();
+    const uint32_t begin = (uint32_t)chunk + threadIdx.x;
+    uint32_t key[kSideItems];
 #pragma unroll
-  for (uint32_t r = 0; r < kSideItems; ++r) {
-    const uint32_t i = begin + r * 256;
-    key[r] = i < n ? keys[i] : kSideBins;
+    for (uint32_t r = 0; r < kSideItems; ++r) {
+      const uint32_t i = begin + r * 256;
+      key[r] = i < n ? keys[i] : kSideBins;
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < kSideItems; ++r)
+      if (key[r] < kSideBins) atomicAdd(&next[key[r]], 1u);
+    __syncthreads();
+    if (threadIdx.x < kSideBins) {
+      const uint32_t mine = next[bin];
+      next[bin] = before + (mine ? atomicAdd(&cursors[bin], mine) : 0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < kSideItems; ++r)
+      if (key[r] < kSideBins) order[atomicAdd(&next[key[r]], 1u)] = begin + r * 256;
+    __syncthreads();  // the next chunk's counts
   }
-#pragma unroll
-  for (uint32_t r = 0; r < kSideItems; ++r)
-    if (key[r] < kSideBins) atomicAdd(&next[key[r]], 1u);
-  __syncthreads();
-  if (threadIdx.x < kSideBins) {
-    // lane l has bin kSideBins - 1 - l: the jobs of the bins above it
-    const uint32_t bin = kSideBins - 1 - threadIdx.x, count = counts[bin];
-    const uint32_t before = WaveInclusiveSum(count) - count;
-    const uint32_t mine = next[bin];
-    next[bin] = before + (mine ? atomicAdd(&cursors[bin], mine) : 0);
-  }
-  __syncthreads();
-#pragma unroll
-  for (uint32_t r = 0; r < kSideItems; ++r)
-    if (key[r] < kSideBins) order[atomicAdd(&next[key[r]], 1u)] = begin + r * 256;
 }
 
 __global__ void ConvertSeedsKernel(size_t size, const uint32_t *seed_positions,
@@ -1626,7 +1633,8 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
     // second list is written after the first ring
     uint8_t *keys = (uint8_t *)w.overflow_list;
     uint32_t *counts = w.counters + 8;
-    const dim3 grid(GridFor(size, kSideChunk));
+    // the kernels stride over the chunks that the resident blocks do not take
+    const dim3 grid(GridFor(size, kSideChunk, kResidentBlocks));
     hipLaunchKernelGGL((SideBinsKernel<kReverse>), grid, dim3(256), 0, s, (uint32_t)size, d_q,
                        P.queries, P.delim, keys, counts);
     hipLaunchKernelGGL(SideOrderKernel, grid, dim3(256), 0, s, (uint32_t)size, keys, counts,

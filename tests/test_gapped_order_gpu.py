@@ -80,3 +80,51 @@ def test_order_with_another_delimiter():
     one = extend(q, d, qpos, dpos, False, 31, "grid")
     pick = rng.integers(0, qpos.size, WAVE_JOBS + 999)
     assert np.array_equal(one[pick], extend(q, d, qpos[pick], dpos[pick], False, 31, "grid"))
+
+
+# past what the order kernels' resident blocks take at once (2,048 chunks of
+# 4,096), and past 262,140 chunks, where a grid of one chunk per block ended
+@pytest.mark.parametrize("n", [2048 * 4096 + 4097, 262140 * 4096 + 4097])
+def test_order_of_large_calls(n):
+    L, rng, piece = gz.lib(), np.random.default_rng(7), 1 << 22
+    q, d, qpos, dpos = pairs(rng, rng.integers(1, 60, 1000))
+    print("order: jobs", n, flush=True)
+    m, nl = gz.blosum62()
+    one = extend(q, d, qpos, dpos, False, DELIM, "grid")
+    pick = rng.integers(0, qpos.size, piece)
+    want = one[pick]
+    _, pq = gz.pack_on_device(q)
+    _, pd = gz.pack_on_device(d)
+    dm = gz.DeviceBuffer.from_array(m)
+    s = gz.Stream()
+    arrays = [gz.DeviceBuffer(4 * n) for _ in range(3)]
+
+    def pieces():
+        for at in range(0, n, piece):
+            yield min(piece, n - at), [ctypes.c_void_p(b.ptr.value + 4 * at) for b in arrays]
+
+    # scores that no job has, so that a job left out is seen
+    start = [qpos[pick], dpos[pick], np.full(piece, 0xdeadbeef, np.uint32)]
+    for k, at in pieces():
+        for a, p in zip(start, at):
+            gz.check(L.gz_memcpy_async(p, gz.ptr(a), 4 * k, s.handle))
+    s.sync()
+    h = ctypes.c_void_p()
+    gz.check(L.gz_gapped_extender_create(ctypes.byref(h)))
+    gz.check(L.gz_gapped_extender_set_queries(h, DELIM, pq.ptr))
+    gz.check(L.gz_gapped_extender_set_database(h, pd.ptr))
+    gz.check(L.gz_gapped_extender_set_score_parameters(h, dm.ptr, nl, 11, 1, 26))
+    gz.check(L.gz_gapped_extender_set_max_sequence_length(h, 62))
+    gz.check(L.gz_gapped_extender_extend_one_side_score_only_async(
+        h, n, 0, None, None, None, arrays[0].ptr, arrays[1].ptr, arrays[2].ptr, s.handle))
+    s.sync()
+    f = (ctypes.c_uint32 * 1)()
+    gz.check(L.gz_gapped_extender_failures(h, f))
+    L.gz_gapped_extender_destroy(h)
+    assert f[0] == 0
+    got = [np.empty(piece, np.uint32) for _ in arrays]
+    for k, at in pieces():
+        for a, p, w in zip(got, at, (1, 2, 0)):
+            gz.check(L.gz_memcpy_async(gz.ptr(a), p, 4 * k, s.handle))
+            s.sync()
+            assert np.array_equal(a[:k], want[:k, w])
