@@ -1481,11 +1481,17 @@ constexpr uint32_t kWideSlots = 256;
 constexpr uint32_t kWideSlotsMax = 16384;
 constexpr size_t kWideBudget = (size_t)8 << 30;
 
-inline uint32_t WideSlotsFor(uint32_t wide) {
-  const size_t per = (size_t)(wide ? wide : 1) * (sizeof(int2) + 1);
-  size_t n = kWideBudget / per;
-  n = n < kWideSlots ? kWideSlots : (n > kWideSlotsMax ? kWideSlotsMax : n);
-  return (uint32_t)(n / 64 * 64);
+// Lanes that a call of `size` jobs can use, and the ring's columns for them:
+// neither falls when the jobs or the longest query grow, so a ring of
+// RingColumns(size, wide) serves every call of up to `size` jobs and `wide`
+// columns, whichever form it takes.
+inline size_t RingLanes(size_t size) {
+  const size_t by_jobs = (size + 63) / 64 * 64;
+  return std::max<size_t>(kWideSlots, std::min<size_t>(kWideSlotsMax, by_jobs));
+}
+inline size_t RingColumns(size_t size, uint32_t wide) {
+  const size_t budget = kWideBudget / (sizeof(int2) + 1);
+  return std::max((size_t)kWideSlots * wide, std::min(budget, RingLanes(size) * wide));
 }
 
 enum : int { kWaveAuto = 0, kWaveNever = 1, kWaveDirect = 2 };
@@ -1524,8 +1530,7 @@ struct gz_gapped_extender_s {
   size_t overflow_capacity = 0;
   int2 *wide_cells = nullptr;
   uint8_t *wide_codes = nullptr;
-  uint32_t wide_allocated = 0;
-  uint32_t wide_slots = 0;  // lanes of the allocated global ring
+  size_t ring_columns = 0;  // of the allocated global ring, over all its lanes
   // the failure counter of the last run (its own workspace's, or the
   // allocation-free entry point's scratch on the device it ran on)
   uint32_t *failure_counter = nullptr;
@@ -1598,8 +1603,8 @@ gz_status gz_gapped_extender_convert_to_gapped_extension_seeds_async(
 
 extern "C++" {
 // Device memory one gapped run uses beyond its jobs: the counters (as in the
-// handle), the two overflow lists (room for every job) and the global ring (kWideSlots
-// slots of `wide` cells and codes).
+// handle), the two overflow lists (room for every job) and the global ring
+// (wide_slots lanes of `wide` cells and codes).
 struct GappedWork {
   uint32_t *counters;
   uint32_t *overflow_list, *overflow_list2;
@@ -1777,26 +1782,16 @@ static gz_status GappedReserve(gz_gapped_extender_t h, size_t size, hipStream_t 
     GZ_HIP_CHECK(gz::Malloc(&h->overflow_list2, cap * sizeof(uint32_t)));
     h->overflow_capacity = cap;
   }
-  // lanes: one per job at most, at least kWideSlots, within the budget; a
-  // call that runs on the row kernel leaves the global ring next to nothing
-  // (bands past 128 columns)
-  const bool rows = h->wave_mode == kWaveAuto && size <= RowJobsFor(h->wide) &&
-                    WaveDpServes(h->cutoff, h->gap_open, h->gap_ext);
-  const size_t by_jobs = rows ? 0 : (size + 63) / 64 * 64;
-  const uint32_t want = (uint32_t)std::max<size_t>(
-      kWideSlots, std::min<size_t>(WideSlotsFor(h->wide), by_jobs));
-  if (h->wide_allocated < h->wide || h->wide_slots < want) {
+  const size_t columns = RingColumns(size, h->wide);
+  if (h->ring_columns < columns) {
     if (h->wide_cells) GZ_HIP_CHECK(gz::Free(h->wide_cells));
     if (h->wide_codes) GZ_HIP_CHECK(gz::Free(h->wide_codes));
     h->wide_cells = nullptr;
     h->wide_codes = nullptr;
-    h->wide_allocated = 0;
-    h->wide_slots = 0;
-    const uint32_t slots = want;
-    GZ_HIP_CHECK(gz::Malloc(&h->wide_cells, (size_t)slots * h->wide * sizeof(int2)));
-    GZ_HIP_CHECK(gz::Malloc(&h->wide_codes, (size_t)slots * h->wide));
-    h->wide_allocated = h->wide;
-    h->wide_slots = slots;
+    h->ring_columns = 0;
+    GZ_HIP_CHECK(gz::Malloc(&h->wide_cells, columns * sizeof(int2)));
+    GZ_HIP_CHECK(gz::Malloc(&h->wide_codes, columns));
+    h->ring_columns = columns;
   }
   return GZ_OK;
 }
@@ -1815,8 +1810,9 @@ static gz_status GappedRun(gz_gapped_extender_t h, size_t size, int reverse,
   // are kept until gz_gapped_extender_failures reads them
   hipLaunchKernelGGL(ResetRunCountersKernel, dim3(1), dim3(256), 0, s, h->counters, 0);
   GZ_HIP_CHECK(hipGetLastError());
+  const size_t lanes = std::min(RingLanes(size), h->ring_columns / h->wide / 64 * 64);
   const GappedWork w = {h->counters,   h->overflow_list, h->overflow_list2, h->wide_cells,
-                        h->wide_codes, h->wide,          h->wide_slots};
+                        h->wide_codes, h->wide,          (uint32_t)lanes};
   h->failure_counter = h->counters + 1;
   return GappedLaunchAll(h, w, size, reverse, d_q, d_d, d_scores, d_cells, s, wide_first, order);
 }

@@ -186,8 +186,10 @@ gz_status gz_gapped_extender_extend_one_side_score_only_cells_async(
 gz_status gz_gapped_extender_set_narrow_ring(gz_gapped_extender_t h, uint32_t columns);
 /* Allocates the extender's workspace for calls of up to `size` jobs now
  * (calls allocate it on demand otherwise), so that a later call allocates
- * nothing and its launch sequence can be captured in a graph.  No reference
- * counterpart. */
+ * nothing and its launch sequence can be captured in a graph.  Holds for
+ * maximum sequence lengths up to the one set by now
+ * (gz_gapped_extender_set_max_sequence_length) and for any other setting.
+ * No reference counterpart. */
 gz_status gz_gapped_extender_reserve(gz_gapped_extender_t h, size_t size, gz_stream_t stream);
 /* persistent != 0: the first ring's extensions run as one persistent launch
  * (as many waves as the device holds) fed from a device work queue: each
