@@ -1622,13 +1622,18 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
   uint32_t *list2_out = w.counters + 4;
   // one wave per job with the row in registers (wave_dp.h), for calls with
   // few jobs and for the bands that outgrow the first ring
-  const bool rows = h->wave_mode == kWaveAuto && WaveDpServes(P.cutoff, P.gap_open, P.gap_ext);
+  const int columns = h->wave_mode == kWaveAuto
+                          ? RowColumnsFor(P.cutoff, P.gap_open, P.gap_ext, w.wide)
+                          : 0;
+  const bool rows = columns > 0;
+  const auto row_kernel =
+      columns == 4 ? GappedRowKernel<kReverse, 4> : GappedRowKernel<kReverse, 2>;
   const WaveDpParams R = {P.queries, P.database, P.delim, P.gap_open + P.gap_ext,
                           P.gap_ext, P.cutoff, kWaveDpMargin};
   const uint32_t *none = nullptr;
 #define GZ_ROWS(N, LIST, COUNT, ORDER, NARROW)                                                  \
-  hipLaunchKernelGGL((GappedRowKernel<kReverse>), dim3(WaveDpBlocksFor(N)), dim3(kWaveDpBlock), \
-                     0, s, (uint32_t)(N), LIST, COUNT, ORDER, (uint32_t)size, R, h->matrix,     \
+  hipLaunchKernelGGL(row_kernel, dim3(WaveDpBlocksFor(N)), dim3(kWaveDpBlock), 0, s,            \
+                     (uint32_t)(N), LIST, COUNT, ORDER, (uint32_t)size, R, h->matrix,           \
                      h->number_letters, d_q, d_d, d_scores, d_cells, list2_out,                 \
                      w.overflow_list2, (int)h->narrow, NARROW, wide_out, failures)
   const bool row_jobs = rows && size <= RowJobsFor(h->wide);

@@ -14,8 +14,8 @@
 // against the lane forms: 300 read extensions 310 -> 25 us, 20,011 of
 // proteins of 100-500 residues 4.0 -> 0.31 ms, 3,001 of Pareto lengths up to
 // 35,000 99.8 -> 10 ms; 1,000,003 of reads (first ring on lanes, its
-// overflow here) 1.38 -> 1.24 ms.  C is 1 and widens to 2 when a band needs
-// it: with one column per lane nothing inside a lane is serial, and bands
+// overflow here) 1.38 -> 1.24 ms.  C is 1 and widens to 2 and 4 when a band
+// needs it: with one column per lane nothing inside a lane is serial, and bands
 // at the presearch's cutoff are 15 to 30 columns wide.  The result build
 // (traceback.hip) records the operations of the same rows, in windows of up
 // to 4 columns per lane at its higher cutoff.
@@ -92,8 +92,35 @@ struct WaveDpParams {
 };
 
 // Margin of the score-only form: what the presearch's parameters (26, 12, 1)
-// need; wider gaps are rare and end in the global ring.
+// need.  Wider gaps are rare: a job that loses a row to one goes to the global
+// ring, or starts again in a wider window in the kernel for four columns.
 constexpr int kWaveDpMargin = 16;
+
+// Most columns per lane that a call's jobs take in the score-only form, 0
+// where lanes are the better form.  `wide`: the longest query side, as the
+// power of two of columns that it is given.
+//   * Two serve sides of up to 62 residues, which end inside the first
+//     window, and cutoffs that pay for few gaps, whose bands stay below 128
+//     columns and whose first row below 64.  The kernel for four
+//     keeps 84 registers instead of 47 and is 2 to 5% slower where two are
+//     enough (20,011 of 100-500 residues at cutoff 26, gaps 11/1: 309 us and 325;
+//     at 42 485 and 497); where they are not, jobs run again on the global
+//     ring (at 46 762 and 553, at 60 1,367 and 648; 3,001 of Pareto lengths
+//     at 60 70 ms and 19).
+//   * Long sides whose bands outgrow 256 columns too pay for both forms, and
+//     the longest one's rows are the call's time: 3,001 of Pareto lengths at
+//     110 88 ms so and 68 on lanes, at 120 94 and 73, at 100 32 and 65; 3,000 of
+//     2,000-4,000 residues at 120 9.9 and 9.3.  Shorter sides gain anyway (3,000
+//     of 1,000-2,000 at 120 4.2 and 5.5).
+inline int RowColumnsFor(int cutoff, int gap_open, int gap_ext, uint32_t wide) {
+  if (!WaveDpServes(cutoff, gap_open, gap_ext)) return 0;
+  const int gap_init = gap_open + gap_ext;
+  if (wide <= 64 || cutoff < gap_init) return 2;
+  if (gap_ext == 0) return 4;
+  const int span = (cutoff - gap_init) / gap_ext + 1;  // columns that one gap can pass
+  if (wide > 2048 && span * cutoff > 800 * gap_init) return 0;
+  return span > 16 && 2 * cutoff > 7 * gap_init ? 4 : 2;
+}
 
 // The value of a wave-uniform expression as a scalar.
 __device__ __forceinline__ int Uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -491,6 +518,16 @@ struct WaveDp {
     ReadWindow(P, B, kWave * H);
     Limits(B);
   }
+
+  // Goes on from a narrower window that ended with r: at its row, or from the
+  // seed when it lost that row.
+  __device__ __forceinline__ int TakeOver(const WaveDpParams &P, WaveDpBand &B,
+                                          const WaveDp<kReverse, C / 2> &x, int r, uint32_t q,
+                                          uint32_t dp) {
+    if (r != kWaveDpWiden) return Begin(P, B, q, dp);
+    Widen(P, B, x);
+    return 0;
+  }
 };
 
 // No operations recorded.
@@ -540,10 +577,10 @@ struct BlockJobs {
 
 // One wave per job: jobs k (order[k] when `order` is set), or the
 // *list_count jobs of `list` when that is set and they are at most
-// kWaveDpJobs.  A job whose band outgrows 128 columns is appended to
-// overflow_list; narrow_count and wide_count (either may be null) count those
-// past narrow_columns and past 64 columns.
-template <bool kReverse>
+// kWaveDpJobs.  A job whose band outgrows 64 kMostColumns columns is appended
+// to overflow_list; narrow_count and wide_count (either may be null) count
+// those past narrow_columns and past 64 columns.
+template <bool kReverse, int kMostColumns>
 __global__ void __launch_bounds__(kWaveDpBlock)
     GappedRowKernel(uint32_t n, const uint32_t *list, const uint32_t *list_count,
                     const uint32_t *order, uint32_t limit, WaveDpParams P, const int *matrix,
@@ -576,11 +613,21 @@ __global__ void __launch_bounds__(kWaveDpBlock)
     NoOps none;
     int r = x.Begin(P, B, q, d);
     if (r == 0) r = x.Rows(P, sm, B, none);
-    if (r == kWaveDpWiden) {
-      // two columns per lane from here on
+    if constexpr (kMostColumns == 2) {
+      if (r == kWaveDpWiden) {
+        WaveDp<kReverse, 2> y;
+        y.Widen(P, B, x);
+        r = y.Rows(P, sm, B, none);
+      }
+    } else if (r != kWaveDpDone) {
       WaveDp<kReverse, 2> y;
-      y.Widen(P, B, x);
-      r = y.Rows(P, sm, B, none);
+      r = y.TakeOver(P, B, x, r, q, d);
+      if (r == 0) r = y.Rows(P, sm, B, none);
+      if (r != kWaveDpDone) {
+        WaveDp<kReverse, 4> z;
+        r = z.TakeOver(P, B, y, r, q, d);
+        if (r == 0) r = z.Rows(P, sm, B, none);
+      }
     }
     if (leads) {
       const bool done = r == kWaveDpDone;

@@ -30,7 +30,7 @@ def pairs(rng, lengths, identity, indel):
     return q, d, (qo[:-1] + k).astype(np.uint32), (do[:-1] + k).astype(np.uint32)
 
 
-def extend(q, d, qpos, dpos, reverse, cutoff, gap_open=11, gap_ext=1, order=None):
+def extend(q, d, qpos, dpos, reverse, cutoff, gap_open=11, gap_ext=1, order=None, told=4000):
     L, n = gz.lib(), qpos.size
     m, nl = gz.blosum62()
     _, pq = gz.pack_on_device(q)
@@ -41,7 +41,7 @@ def extend(q, d, qpos, dpos, reverse, cutoff, gap_open=11, gap_ext=1, order=None
     gz.check(L.gz_gapped_extender_set_queries(h, DELIM, pq.ptr))
     gz.check(L.gz_gapped_extender_set_database(h, pd.ptr))
     gz.check(L.gz_gapped_extender_set_score_parameters(h, dm.ptr, nl, gap_open, gap_ext, cutoff))
-    gz.check(L.gz_gapped_extender_set_max_sequence_length(h, 4000))
+    gz.check(L.gz_gapped_extender_set_max_sequence_length(h, told))
     s = gz.Stream()
     dq, dd = gz.DeviceBuffer.from_array(qpos), gz.DeviceBuffer.from_array(dpos)
     ds, dc = gz.DeviceBuffer(4 * n), gz.DeviceBuffer(4 * n)
@@ -114,3 +114,27 @@ def test_rows_equal_lanes(cutoff, reverse):
     for a, b, c in zip(one, many, turned):
         assert np.array_equal(a[pick], b)
         assert np.array_equal(a, c)
+
+
+# the two- and the four-column kernel and what decides between them and the
+# lanes: sides around 126 and 254 residues and past 2,046 told, bands that
+# start past 64 columns, lose a row to a gap and outgrow 128 and 256
+@pytest.mark.parametrize("cutoff,gap_open,gap_ext", [
+    (26, 11, 1), (26, 5, 1), (42, 11, 1), (43, 11, 1), (73, 11, 1), (74, 11, 1), (90, 11, 1),
+    (99, 11, 1), (105, 11, 1), (120, 11, 1), (120, 0, 1), (26, 11, 0), (60, 0, 0), (60, 2, 3),
+    (120, 500, 12)])
+@pytest.mark.parametrize("told,lengths", [
+    (62, (1, 40, 60, 61, 62)), (126, (63, 64, 100, 124, 125, 126)),
+    (2046, (126, 127, 128, 129, 253, 254, 255, 256, 257, 700)), (2047, (300, 2047))])
+@pytest.mark.parametrize("reverse", [False, True])
+def test_windows_vs_oracle(told, lengths, cutoff, gap_open, gap_ext, reverse):
+    rng = np.random.default_rng(told + 7 * cutoff + gap_open)
+    print("windows: told", told, "cutoff", cutoff, "gaps", gap_open, gap_ext, reverse, flush=True)
+    q, d, qpos, dpos = pairs(rng, np.repeat(lengths, 8), (0.25, 1.0), 0.05)
+    if reverse:
+        qpos, dpos = qpos - 1, dpos - 1
+    s, qe, de, _ = extend(q, d, qpos, dpos, reverse, cutoff, gap_open, gap_ext, told=told)
+    want = oracle(q, d, qpos, dpos, reverse, cutoff, gap_open, gap_ext)
+    got = np.stack([s, qe, de], 1).astype(np.int64)
+    bad = np.nonzero((got != want).any(1))[0]
+    assert bad.size == 0, (bad[:5], got[bad[:5]], want[bad[:5]])
