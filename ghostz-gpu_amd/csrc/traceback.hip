@@ -535,14 +535,11 @@ __device__ void WaveSide(const WaveDpParams &P, const int8_t *sm, uint32_t q0, u
       WaveDp<kReverse, 2> y;
       r = y.Begin(P, B, q0, d0);
       if (r == 0) r = y.Rows(P, sm, B, ops);
-      if (r == kWaveDpWiden || (r == kWaveDpLost && B.row == 0 && !ops.full)) {
+      if (r != kWaveDpDone && !ops.full) {
+        // a lost row's side starts again, its operations with it
         WaveDp<kReverse, 4> z;
-        if (r == kWaveDpWiden) {
-          z.Widen(P, B, y);
-          r = 0;
-        } else {
-          r = z.Begin(P, B, q0, d0);
-        }
+        if (r == kWaveDpLost) ops.used = 0;
+        r = z.TakeOver(P, B, y, r, q0, d0);
         if (r == 0) r = z.Rows(P, sm, B, ops);
       }
     }
@@ -861,10 +858,7 @@ hipError_t TracebackRunner::Queue(const TracebackInputs &in, const TracebackJob 
   uint32_t listed = 0;
   if (waves) {
     const WaveDpParams P = {in.queries, in.database, kDelimiter, in.gap_open + in.gap_ext,
-                            in.gap_ext, in.cutoff,
-                            in.gap_ext > 0 ? std::max(in.cutoff - in.gap_open - in.gap_ext, 0) /
-                                                 in.gap_ext + 2
-                                           : kWaveDpMargin};
+                            in.gap_ext, in.cutoff, kWaveDpMargin};
     hipLaunchKernelGGL(ClearKernel, dim3(1), dim3(64), 0, s, d_counters, 3u);
     hipLaunchKernelGGL(TracebackWaveKernel, dim3(2 * side_blocks), dim3(kTbWaveBlock), 0, s, P,
                        d_jobs, n, batch, d_counters, in.matrix, in.nl, scratch, wc, d_halves);

@@ -116,6 +116,27 @@ def test_waves_vs_oracle(cutoff, gap_open, gap_ext):
     assert served > len(jobs) // 2
 
 
+@pytest.mark.parametrize("cutoff,gap_open,gap_ext", [
+    (70, 11, 1), (90, 11, 1), (99, 11, 1), (60, 6, 1), (52, 11, 0), (120, 2, 3)])
+def test_wide_bands_vs_oracle(cutoff, gap_open, gap_ext):
+    """Rows that a gap fills past the window: the side starts again in the
+    wider one, sides that the widest one ends and sides that it does not."""
+    rng = np.random.default_rng(cutoff + gap_open)
+    print("traceback wide bands: cutoff", cutoff, "gaps", gap_open, gap_ext, flush=True)
+    q, d, jobs, most = jobs_of(rng, np.repeat((120, 200, 252, 255, 256, 260, 300), 12), (0.3, 1.0),
+                               0.04, 0.0)
+    out = build(q, d, jobs, most, cutoff, gap_open, gap_ext)
+    served = 0
+    for k, job in enumerate(jobs):
+        if out[k, 9]:
+            continue
+        served += 1
+        got = tuple(int(x) for x in out[k, :6].astype(np.int64))
+        want = by_oracle(q, d, job, cutoff, gap_open, gap_ext)
+        assert got == want, (k, job, got, want)
+    assert served > len(jobs) // 2
+
+
 def test_more_jobs_than_waves():
     """Jobs past the resident waves' first ones, and their order in the call."""
     rng = np.random.default_rng(5)
