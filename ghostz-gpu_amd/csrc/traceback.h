@@ -45,10 +45,15 @@ class TracebackRunner {
  private:
   hipError_t Queue(const TracebackInputs &in, const TracebackJob *jobs, uint32_t n,
                    TracebackOut *outs, hipStream_t s, float *kernel_ms);
-  hipError_t Reserve(size_t bytes);
-  // one lane per job (d_list: the n jobs to run)
+  hipError_t Reserve(size_t bytes, void **p, size_t *capacity);
+  void Release(void **p, size_t *capacity);
+  // `before` bytes and the lanes' scratch, for fewer lanes while memory lacks
+  hipError_t ReserveLanes(size_t before, size_t lanes, size_t bytes_per_lane, void **p,
+                          size_t *capacity);
+  // one lane per job (d_list: the n jobs to run), as many as `bytes` of scratch hold
   hipError_t Lanes(const TracebackInputs &in, const TracebackJob *d_jobs, uint32_t n,
-                   const uint32_t *d_list, TracebackOut *d_outs, hipStream_t s);
+                   const uint32_t *d_list, TracebackOut *d_outs, uint8_t *scratch, size_t bytes,
+                   hipStream_t s);
   const bool pooled_;
   void *ws_ = nullptr, *lane_ws_ = nullptr;
   size_t cap_ = 0, lane_cap_ = 0;

@@ -730,6 +730,14 @@ LaneCaps TracebackCaps(uint32_t max_query_length, uint32_t max_subject_length) {
   return c;
 }
 
+// Lanes of n results: those resident at once (up to seven 64-lane blocks per
+// CU), within a 12 GB scratch budget.
+size_t TracebackLanes(uint32_t n, const LaneCaps &caps) {
+  const size_t budget = (size_t)12 << 30;
+  const size_t lanes = std::min<size_t>(((size_t)n + 63) / 64 * 64, (size_t)7 * 64 * 256);
+  return std::max<size_t>(64, std::min(lanes, budget / caps.bytes_per_lane / 64 * 64));
+}
+
 // A wave's: an arena that holds the rows a side can have, up to the limit.
 WaveCaps TracebackWaveCaps(uint32_t max_query_length, uint32_t max_subject_length) {
   WaveCaps c;
@@ -746,62 +754,62 @@ WaveCaps TracebackWaveCaps(uint32_t max_query_length, uint32_t max_subject_lengt
 }  // namespace
 
 TracebackRunner::~TracebackRunner() {
-  if (ws_ && pooled_) WorkspacePool::Give(ws_, cap_);
-  else if (ws_) (void)gz::Free(ws_);
-  if (lane_ws_) (void)gz::Free(lane_ws_);
+  Release(&ws_, &cap_);
+  Release(&lane_ws_, &lane_cap_);
   for (hipEvent_t e : ev_)
     if (e) (void)hipEventDestroy(e);
 }
 
-hipError_t TracebackRunner::Reserve(size_t bytes) {
-  if (cap_ >= bytes) return hipSuccess;
-  if (ws_ && pooled_) WorkspacePool::Give(ws_, cap_);
-  else if (ws_) (void)gz::Free(ws_);
-  ws_ = nullptr;
-  cap_ = 0;
+void TracebackRunner::Release(void **p, size_t *capacity) {
+  if (*p && pooled_) WorkspacePool::Give(*p, *capacity);
+  else if (*p) (void)gz::Free(*p);
+  *p = nullptr;
+  *capacity = 0;
+}
+
+hipError_t TracebackRunner::Reserve(size_t bytes, void **p, size_t *capacity) {
+  if (*capacity >= bytes) return hipSuccess;
+  Release(p, capacity);
   hipError_t e;
   if (pooled_) {
-    e = WorkspacePool::Take(bytes, &ws_, &cap_);
+    e = WorkspacePool::Take(bytes, p, capacity);
   } else {
-    e = gz::Malloc(&ws_, bytes);
-    cap_ = bytes;
+    e = gz::Malloc(p, bytes);
+    *capacity = bytes;
   }
   if (e != hipSuccess) {
-    ws_ = nullptr;
-    cap_ = 0;
+    *p = nullptr;
+    *capacity = 0;
   }
   return e;
 }
 
+hipError_t TracebackRunner::ReserveLanes(size_t before, size_t lanes, size_t bytes_per_lane,
+                                         void **p, size_t *capacity) {
+  for (;;) {
+    const hipError_t e = Reserve(before + lanes * bytes_per_lane, p, capacity);
+    if (e != hipErrorOutOfMemory || lanes <= 64) return e;
+    (void)hipGetLastError();
+    lanes = lanes / 2 / 64 * 64;
+  }
+}
+
 hipError_t TracebackRunner::Lanes(const TracebackInputs &in, const TracebackJob *d_jobs,
                                   uint32_t n, const uint32_t *d_list, TracebackOut *d_outs,
-                                  hipStream_t s) {
+                                  uint8_t *scratch, size_t bytes, hipStream_t s) {
   const LaneCaps caps = TracebackCaps(in.max_query_length, in.max_subject_length);
-  // lanes resident at once (up to seven 64-lane blocks per CU), bounded by a
-  // 12 GB scratch budget
-  const size_t budget = (size_t)12 << 30;
-  size_t lanes = std::min<size_t>(((size_t)n + 63) / 64 * 64, (size_t)7 * 64 * 256);
-  lanes = std::max<size_t>(64, std::min(lanes, budget / caps.bytes_per_lane / 64 * 64));
-  const size_t bytes = lanes * caps.bytes_per_lane;
-  if (lane_cap_ < bytes) {
-    if (lane_ws_) (void)gz::Free(lane_ws_);
-    lane_ws_ = nullptr;
-    lane_cap_ = 0;
-    const hipError_t e = gz::Malloc(&lane_ws_, bytes);
-    if (e != hipSuccess) return e;
-    lane_cap_ = bytes;
-  }
+  const size_t lanes = std::min(TracebackLanes(n, caps), bytes / caps.bytes_per_lane / 64 * 64);
   const uint32_t blocks = (uint32_t)(lanes / kTbThreads);
   const bool short_cells =
       in.cutoff <= 8192 && in.gap_ext >= 0 && in.gap_open + in.gap_ext <= 1024;
   if (short_cells)
     hipLaunchKernelGGL(TracebackKernel<true>, dim3(blocks), dim3(kTbThreads), 0, s, in.queries,
                        in.database, d_jobs, n, d_list, in.matrix, in.nl, in.gap_open, in.gap_ext,
-                       in.cutoff, (uint8_t *)lane_ws_, caps, d_outs);
+                       in.cutoff, scratch, caps, d_outs);
   else
     hipLaunchKernelGGL(TracebackKernel<false>, dim3(blocks), dim3(kTbThreads), 0, s, in.queries,
                        in.database, d_jobs, n, d_list, in.matrix, in.nl, in.gap_open, in.gap_ext,
-                       in.cutoff, (uint8_t *)lane_ws_, caps, d_outs);
+                       in.cutoff, scratch, caps, d_outs);
   return hipGetLastError();
 }
 
@@ -830,11 +838,12 @@ hipError_t TracebackRunner::Queue(const TracebackInputs &in, const TracebackJob 
   uint32_t side_blocks = 0, batch = 1;
   if (waves) {
     wc = TracebackWaveCaps(in.max_query_length, in.max_subject_length);
-    // waves of a side: as many as jobs up to half the resident ones, within
-    // a 4 GB scratch budget
-    uint64_t side_waves = std::min<uint64_t>(n, kTbWaves / 2);
-    side_waves = std::min<uint64_t>(side_waves, ((uint64_t)4 << 30) / 2 / wc.stride);
-    side_blocks = (uint32_t)std::max<uint64_t>(1, (side_waves + per - 1) / per);
+    // blocks of a side: for as many waves as jobs up to half the resident
+    // ones, within a 4 GB scratch budget, but at least one (subjects of tens
+    // of millions of residues: up to 10 GB)
+    const uint64_t side_waves = std::min<uint64_t>(n, kTbWaves / 2);
+    const uint64_t fit = ((uint64_t)4 << 30) / 2 / ((uint64_t)per * wc.stride);
+    side_blocks = (uint32_t)std::max<uint64_t>(1, std::min((side_waves + per - 1) / per, fit));
     const uint64_t b = n / ((uint64_t)side_blocks * per * 8) + 1;
     batch = (uint32_t)std::min<uint64_t>(b, 4);
   }
@@ -842,8 +851,11 @@ hipError_t TracebackRunner::Queue(const TracebackInputs &in, const TracebackJob 
   const size_t a_outs = Align256(n * sizeof(TracebackOut));
   const size_t a_half = waves ? Align256(2 * (size_t)n * sizeof(TracebackHalf)) : 0;
   const size_t a_list = waves ? Align256((size_t)n * 4) : 0;
-  const size_t a_wave = (size_t)side_blocks * 2 * per * wc.stride;
-  hipError_t e = Reserve(a_jobs + a_outs + 256 + a_half + a_list + a_wave);
+  const size_t before = a_jobs + a_outs + 256 + a_half + a_list;
+  const LaneCaps lc = TracebackCaps(in.max_query_length, in.max_subject_length);
+  hipError_t e = waves ? Reserve(before + (size_t)side_blocks * 2 * per * wc.stride, &ws_, &cap_)
+                       : ReserveLanes(before, TracebackLanes(n, lc), lc.bytes_per_lane, &ws_,
+                                      &cap_);
   if (e != hipSuccess) return e;
   char *w = (char *)ws_;
   TracebackJob *d_jobs = (TracebackJob *)w;
@@ -851,7 +863,7 @@ hipError_t TracebackRunner::Queue(const TracebackInputs &in, const TracebackJob 
   uint32_t *d_counters = (uint32_t *)(w + a_jobs + a_outs);  // heads, listed jobs
   TracebackHalf *d_halves = (TracebackHalf *)(w + a_jobs + a_outs + 256);
   uint32_t *d_list = (uint32_t *)(w + a_jobs + a_outs + 256 + a_half);
-  uint8_t *scratch = (uint8_t *)(w + a_jobs + a_outs + 256 + a_half + a_list);
+  uint8_t *scratch = (uint8_t *)(w + before);
   e = hipMemcpyAsync(d_jobs, jobs, n * sizeof(TracebackJob), hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipEventRecord(ev_[0], s);
   if (e != hipSuccess) return e;
@@ -866,7 +878,7 @@ hipError_t TracebackRunner::Queue(const TracebackInputs &in, const TracebackJob 
                        d_halves, d_outs, d_counters + 2, d_list);
     e = hipGetLastError();
   } else {
-    e = Lanes(in, d_jobs, n, nullptr, d_outs, s);
+    e = Lanes(in, d_jobs, n, nullptr, d_outs, scratch, cap_ - before, s);
   }
   if (e == hipSuccess) e = hipEventRecord(ev_[1], s);
   // the copies back are queued once the kernels are done: a device-to-host
@@ -876,8 +888,21 @@ hipError_t TracebackRunner::Queue(const TracebackInputs &in, const TracebackJob 
     e = hipMemcpyAsync(&listed, d_counters + 2, 4, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e == hipSuccess && listed > 0) {
-      // bands past 256 columns and jobs whose frame is not as described
-      e = Lanes(in, d_jobs, listed, d_list, d_outs, s);
+      // bands past 256 columns and jobs whose frame is not as described, in
+      // the waves' scratch, which is idle by now, where it has room for them
+      const size_t lanes = TracebackLanes(listed, lc);
+      size_t bytes = cap_ - before;
+      if (bytes < lanes * lc.bytes_per_lane) {
+        e = ReserveLanes(0, lanes, lc.bytes_per_lane, &lane_ws_, &lane_cap_);
+        if (e == hipSuccess) {
+          scratch = (uint8_t *)lane_ws_;
+          bytes = lane_cap_;
+        } else if (bytes >= 64 * lc.bytes_per_lane) {
+          (void)hipGetLastError();
+          e = hipSuccess;
+        }
+      }
+      if (e == hipSuccess) e = Lanes(in, d_jobs, listed, d_list, d_outs, scratch, bytes, s);
       if (e == hipSuccess) e = hipEventRecord(ev_[1], s);
       if (e == hipSuccess) e = hipEventSynchronize(ev_[1]);
     }

@@ -2,6 +2,7 @@
 result build and the CPU oracle.  All fields are whole numbers and are
 compared exactly; a result that reads a byte an earlier extension left must be
 flagged as the host flags it."""
+import ctypes
 import threading
 
 import numpy as np
@@ -167,6 +168,36 @@ def test_bounds_of_the_call():
     part = jobs.copy()
     part[:, 1] -= 3  # the frame ends before the query's delimiter
     assert np.array_equal(build(q, d, part, most, 52), full)
+
+
+def free_bytes():
+    hip = ctypes.CDLL("libamdhip64.so")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("lengths,n", [((20, 60), 9001), ((200, 400), 3001), ((200, 400), 33)])
+def test_jobs_off_the_waves(lengths, n):
+    """Jobs that take a lane each, in the waves' scratch where it has room for
+    them (long sides) and in a block of their own where not (short ones): all,
+    some and one of a call, and a cutoff that the waves do not serve.  Between
+    calls no more is kept than the pool's 512 MB."""
+    rng = np.random.default_rng(n)
+    q, d, jobs, most = jobs_of(rng, rng.integers(*lengths, 200), (0.4, 1.0), 0.04)
+    jobs = jobs[rng.integers(0, len(jobs), n)]
+    print("traceback lanes: jobs", n, "lengths", lengths, flush=True)
+    before = free_bytes()
+    full = build(q, d, jobs, most, 52)
+    for every in (1, 40, n):
+        part = jobs.copy()
+        part[::every, 1] -= 1  # the frame ends before the query's delimiter
+        assert np.array_equal(build(q, d, part, most, 52), full)
+    large = build(q, d, jobs, most, 130)
+    assert np.array_equal(large[:20], np.concatenate(
+        [build(q, d, jobs[k:k + 1], most, 130, max_query=int(jobs[:, 1].max()))
+         for k in range(20)]))
+    assert before - free_bytes() <= (512 << 20) + (64 << 20)  # and the runtime's own
 
 
 def test_concurrent_calls():
