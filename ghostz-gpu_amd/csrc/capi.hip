@@ -97,6 +97,11 @@ bool gz::WorkspacePool::Trim() {
   return any;
 }
 
+extern "C" gz_status gz_release_workspaces(void) {
+  (void)gz::WorkspacePool::Trim();
+  return GZ_OK;
+}
+
 struct gz_aligner_s {
   std::vector<int> matrix;
   AlignerOptions opt;

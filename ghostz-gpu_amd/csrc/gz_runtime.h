@@ -23,7 +23,7 @@ std::recursive_mutex &CaptureLock();
 // block, is its only user until its kernels and copies have ended, and gives
 // it back; one block per device is kept between calls, of at most kMost
 // bytes, the largest given back (a call that finds none, or one too small,
-// allocates its own).  Mapping and unmapping a call's scratch costs far more
+// allocates its own; gz_release_workspaces frees them).  Mapping and unmapping a call's scratch costs far more
 // than using it: 50,021 read results (140 MB of scratch) take 11 ms with an
 // allocation per call and 1.34 ms without where other allocations of the
 // process come and go, 3,001 protein results (300 MB) 12 and 0.67 ms.

@@ -31,6 +31,7 @@ _SIGNATURES = {
     "gz_stream_create": (c_int, [POINTER(c_void_p)]),
     "gz_stream_destroy": (c_int, [c_void_p]),
     "gz_stream_synchronize": (c_int, [c_void_p]),
+    "gz_release_workspaces": (c_int, []),
     "gz_memcpy_async": (c_int, [c_void_p, c_void_p, c_size_t, c_void_p]),
     "gz_memset_async": (c_int, [c_void_p, c_int, c_size_t, c_void_p]),
     "gz_copy_kernel_async": (c_int, [c_void_p, c_void_p, c_size_t, c_void_p]),

@@ -40,6 +40,12 @@ const char *gz_last_error(void);
 gz_status gz_set_device(int device);                 /* cudaSetDevice */
 gz_status gz_device_malloc(void **ptr, size_t bytes);
 gz_status gz_device_free(void *ptr);
+/* Frees the device workspaces that the library keeps between calls without a
+ * handle of their own (gz_build_results) or with a training set
+ * (gz_mlp_train_epochs): one block per GPU of at most 512 MB, which is also
+ * given up when an allocation of the library fails.  Safe at any time; calls
+ * in flight keep their blocks.  To be called before a hipDeviceReset. */
+gz_status gz_release_workspaces(void);
 gz_status gz_host_malloc(void **ptr, size_t bytes);  /* pinned */
 gz_status gz_host_free(void *ptr);
 gz_status gz_stream_create(gz_stream_t *stream);

@@ -200,6 +200,19 @@ def test_jobs_off_the_waves(lengths, n):
     assert before - free_bytes() <= (512 << 20) + (64 << 20)  # and the runtime's own
 
 
+def test_kept_workspace_is_released():
+    rng = np.random.default_rng(9)
+    q, d, jobs, most = jobs_of(rng, rng.integers(200, 400, 3000), (0.4, 1.0), 0.04)
+    print("traceback: kept workspace", flush=True)
+    gz.check(gz.lib().gz_release_workspaces())
+    want = build(q, d, jobs, most, 52)
+    kept = free_bytes()
+    gz.check(gz.lib().gz_release_workspaces())
+    assert free_bytes() - kept > 100 << 20
+    gz.check(gz.lib().gz_release_workspaces())  # nothing to free
+    assert np.array_equal(build(q, d, jobs, most, 52), want)
+
+
 def test_concurrent_calls():
     """Calls of several threads at once, of different sizes: each has a
     workspace of its own, the kept one or a new one."""
