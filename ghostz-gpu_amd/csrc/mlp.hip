@@ -835,12 +835,12 @@ class Slab {
  public:
   template <typename T>
   void Add(T **p, size_t count) {
-    parts_.push_back({(void **)p, bytes_});
+    parts_[n_++] = {(void **)p, bytes_};
     bytes_ += (count * sizeof(T) + 255) / 256 * 256;
   }
   size_t bytes() const { return bytes_; }
   void Place(void *base) const {
-    for (const Part &x : parts_) *x.p = (char *)base + x.at;
+    for (int i = 0; i < n_; ++i) *parts_[i].p = (char *)base + parts_[i].at;
   }
 
  private:
@@ -848,7 +848,8 @@ class Slab {
     void **p;
     size_t at;
   };
-  std::vector<Part> parts_;
+  Part parts_[8];  // the most that a slab has
+  int n_ = 0;
   size_t bytes_ = 0;
 };
 
