@@ -38,6 +38,9 @@ namespace gz {
 struct GappedTuner {
   static constexpr int kConfigs = 4;
   static constexpr int kTrials = 2;
+  // a bucket that runs one wave per job, where no configuration matters: not
+  // timed, with an executable graph of its own
+  static constexpr int kRows = kConfigs;
   double ms[kLengthBuckets][kConfigs] = {};
   double jobs[kLengthBuckets][kConfigs] = {};
   int trials[kLengthBuckets][kConfigs] = {};
@@ -170,7 +173,7 @@ class Aligner : public PresearchDevice {
   // sequence, updated with each call's arguments
   bool use_graphs_ = true;
   int forced_layout_ = -1;  // GappedTuner layout from GZ_GAPPED_LAYOUT (-1: tuned)
-  hipGraphExec_t graph_exec_[2 * kLengthBuckets * GappedTuner::kConfigs] = {};
+  hipGraphExec_t graph_exec_[2 * kLengthBuckets * (GappedTuner::kConfigs + 1)] = {};
   uint64_t graph_updates_ = 0, graph_instantiations_ = 0;
   hipError_t LaunchCaptured(int slot, hipStream_t s, const std::function<bool()> &launch);
 };

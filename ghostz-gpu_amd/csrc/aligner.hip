@@ -508,18 +508,22 @@ int Aligner::GappedRun(int slot, size_t ci, uint32_t nr, uint32_t nf, uint32_t *
         if (e != hipSuccess) break;
       }
       std::lock_guard<std::mutex> lock(tuner_mutex_);
-      tuned[b] = tuner_.Pick(b);
-      for (int c = 0; c < GappedTuner::kConfigs; ++c)
-        if (tuner_.trials[b][c] < GappedTuner::kTrials) settled = false;
-      if (gz_gapped_extender_set_narrow_ring(gapped, GappedTuner::Narrow(tuned[b])) != GZ_OK ||
-          gz_gapped_extender_set_persistent(gapped, GappedTuner::Persistent(tuned[b])) != GZ_OK)
-        e = hipErrorUnknown;
+      if (GappedRunsRows(gapped, c)) {
+        tuned[b] = GappedTuner::kRows;
+      } else {
+        tuned[b] = tuner_.Pick(b);
+        for (int c = 0; c < GappedTuner::kConfigs; ++c)
+          if (tuner_.trials[b][c] < GappedTuner::kTrials) settled = false;
+        if (gz_gapped_extender_set_narrow_ring(gapped, GappedTuner::Narrow(tuned[b])) != GZ_OK ||
+            gz_gapped_extender_set_persistent(gapped, GappedTuner::Persistent(tuned[b])) != GZ_OK)
+          e = hipErrorUnknown;
+      }
       if (e == hipSuccess) e = hipEventRecord(tune_ev[2 * b], s);
       // the bucket's launch sequence (both sides: counter resets, the
       // first ring, the 64-column ring, the global ring) as one graph
       auto both = [&]() { return side(o, c, 1) && side(nr + o, c, 0); };
       if (e == hipSuccess) {
-        const int key = (x * kLengthBuckets + b) * GappedTuner::kConfigs + tuned[b];
+        const int key = (x * kLengthBuckets + b) * (GappedTuner::kConfigs + 1) + tuned[b];
         if (use_graphs_) e = LaunchCaptured(key, s, both);
         else if (!both()) e = hipErrorUnknown;
       }
@@ -560,7 +564,7 @@ int Aligner::GappedRun(int slot, size_t ci, uint32_t nr, uint32_t nf, uint32_t *
   if (e == hipSuccess) e = hipEventElapsedTime(&ms, ev[0], ev[1]);
   if (e == hipSuccess && order) e = hipEventElapsedTime(&ms2, S.ev_begin, S.ev_end);
   for (int b = 0; b < kLengthBuckets && e == hipSuccess; ++b) {
-    if (tuned[b] < 0) continue;
+    if (tuned[b] < 0 || tuned[b] == GappedTuner::kRows) continue;
     float bm = 0;
     e = hipEventElapsedTime(&bm, tune_ev[2 * b], tune_ev[2 * b + 1]);
     if (e == hipSuccess) {

@@ -1602,6 +1602,17 @@ gz_status gz_gapped_extender_convert_to_gapped_extension_seeds_async(
 }
 
 extern "C++" {
+// Most columns per lane of the handle's calls on the row kernel; 0: lanes.
+static int RowColumns(const gz_gapped_extender_s *h) {
+  return h->wave_mode == kWaveAuto
+             ? RowColumnsFor(h->cutoff, h->gap_open, h->gap_ext, h->wide)
+             : 0;
+}
+
+bool gz::GappedRunsRows(const gz_gapped_extender_s *h, size_t size) {
+  return RowColumns(h) > 0 && size <= RowJobsFor(h->wide);
+}
+
 // Device memory one gapped run uses beyond its jobs: the counters (as in the
 // handle), the two overflow lists (room for every job) and the global ring
 // (wide_slots lanes of `wide` cells and codes).
@@ -1622,9 +1633,7 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
   uint32_t *list2_out = w.counters + 4;
   // one wave per job with the row in registers (wave_dp.h), for calls with
   // few jobs and for the bands that outgrow the first ring
-  const int columns = h->wave_mode == kWaveAuto
-                          ? RowColumnsFor(P.cutoff, P.gap_open, P.gap_ext, w.wide)
-                          : 0;
+  const int columns = RowColumns(h);
   const bool rows = columns > 0;
   const auto row_kernel =
       columns == 4 ? GappedRowKernel<kReverse, 4> : GappedRowKernel<kReverse, 2>;
@@ -1636,7 +1645,7 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
                      (uint32_t)(N), LIST, COUNT, ORDER, (uint32_t)size, R, h->matrix,           \
                      h->number_letters, d_q, d_d, d_scores, d_cells, list2_out,                 \
                      w.overflow_list2, (int)h->narrow, NARROW, wide_out, failures)
-  const bool row_jobs = rows && size <= RowJobsFor(h->wide);
+  const bool row_jobs = GappedRunsRows(h, size);
   if (!order && wide_first == 0 && !row_jobs && size > kRowJobsShort) {
     // the keys and the order lie in the overflow lists: the first ring reads
     // the order and writes the first list, whose keys are read by then; the

@@ -10,7 +10,13 @@ struct gz_stream_s {
   hipStream_t s;
 };
 
+struct gz_gapped_extender_s;
+
 namespace gz {
+
+// Whether a call of `size` jobs with the extender's present settings runs one
+// wave per job (extenders.hip): the first ring's settings then change nothing.
+bool GappedRunsRows(const gz_gapped_extender_s *h, size_t size);
 
 // Stream capture and memory management exclude each other.  Freeing device
 // or pinned memory synchronizes the device, which a capture in flight on

@@ -598,7 +598,7 @@ class Aligner:
 
     def tuner_state(self):
         """The batched form's autotuner: chosen configuration per query-length
-        bucket (-1: not seen), ms per job and trials per (bucket, config)."""
+        bucket (-1: no call with a lane per job), ms per job and trials per (bucket, config)."""
         chosen = np.zeros(4, np.int32)
         ms = np.zeros(16, np.float64)
         trials = np.zeros(16, np.uint32)

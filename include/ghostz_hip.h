@@ -481,7 +481,8 @@ gz_status gz_aligner_set_database(gz_aligner_t a, gz_database_t db);
 gz_status gz_aligner_graph_counts(gz_aligner_t a, uint64_t *instantiations, uint64_t *updates);
 /* The batched form's autotuner (no reference counterpart): per query-length
  * bucket b (<= 128, <= 512, <= 2048, longer residues), chosen[b] = the
- * gapped configuration it uses next (-1: bucket not seen; configuration c:
+ * gapped configuration it uses next (-1: not seen in a call that runs a lane
+ * per job, the only form that a configuration matters to; configuration c:
  * first ring 16 columns when c & 1, else 32; static grid when c & 2, else
  * the persistent work queue), and for each configuration the measured
  * kernel milliseconds per job and trials (4 x 4 arrays, bucket-major).  Any

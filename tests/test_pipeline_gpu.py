@@ -255,3 +255,21 @@ def test_uneven_queries_at_the_batched_shape_match_oracle(matrix):
     db = gz.Database(dn, dr, do)
     run_case("uneven300x5000", q, db, m, nl,
              schedules=(gz.SCHEDULE_PLAIN, gz.SCHEDULE_LEARNED))
+
+
+def test_tuner_times_lane_calls_only():
+    """Buckets that run one wave per job are not timed (no configuration
+    matters to them) and keep one graph; a bucket past that form is."""
+    q, d = synthetic.translated_workload(8, 20000, 24000)
+    queries, db = gz.Queries(*q, translated=True), gz.Database(*d)
+    say("tuner: small blocks and one block")
+    small = gz.Aligner(db, batched=1, pipeline_blocks=8)
+    text, _ = small.align(queries)
+    chosen, _, trials = small.tuner_state()
+    assert (trials == 0).all() and (chosen == -1).all()
+    assert small.graph_counts()[0] == 1
+    large = gz.Aligner(db, batched=1, pipeline_blocks=1)
+    for _ in range(2):
+        assert large.align(queries)[0] == text
+    chosen, _, trials = large.tuner_state()
+    assert trials.sum() == 2 and (chosen >= 0).sum() == 1
