@@ -1,6 +1,7 @@
-"""Calls of more than 65,536 jobs without an order of their own run in one by
-query side length (extenders.hip): the results are those of the same jobs in
-small calls, at sizes around a block's chunk of 4,096, for sides from none to
+"""Calls that run a lane per job (more than 65,536 jobs, or 131,072 when the
+longest query is told above 62 residues) and bring no order of their own run in
+one by query side length (extenders.hip): the results are those of the same
+jobs in small calls, at sizes around a block's chunk of 4,096, for sides from none to
 past the last bin, with an own delimiter, on every entry point that takes
 such calls."""
 import ctypes
@@ -12,7 +13,7 @@ import gz_native as gz
 from helpers import DELIM, concat, mutate, random_protein
 
 pytestmark = pytest.mark.gpu
-WAVE_JOBS = 65536
+WAVE_JOBS = 131072  # of queries told longer than 62 residues
 
 
 def pairs(rng, lengths):
@@ -60,7 +61,7 @@ def extend(q, d, qpos, dpos, reverse, delim, form):
 
 @pytest.mark.parametrize("form", ["grid", "queue", "noalloc"])
 @pytest.mark.parametrize("reverse", [False, True])
-@pytest.mark.parametrize("n", [WAVE_JOBS + 1, 17 * 4096, 17 * 4096 + 1, 200003])
+@pytest.mark.parametrize("n", [WAVE_JOBS + 1, 33 * 4096, 33 * 4096 + 1, 200003])
 def test_order_leaves_results(n, reverse, form):
     rng = np.random.default_rng(n + int(reverse))
     q, d, qpos, dpos = pairs(rng, np.r_[np.arange(1, 140), rng.integers(1, 60, 900)])

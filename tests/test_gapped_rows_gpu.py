@@ -1,6 +1,6 @@
 """The gapped extension with one wave per job and the row in registers
 (wave_dp.h) against the CPU oracle, and against the lane-per-job form that
-calls of more than 65,536 jobs take.  All outputs are whole numbers and are
+calls of more than 131,072 jobs (of queries past 62 residues) take.  All outputs are whole numbers and are
 compared exactly."""
 import ctypes
 
@@ -12,7 +12,7 @@ import oracle_py
 from helpers import DELIM, concat, mutate, random_protein
 
 pytestmark = pytest.mark.gpu
-WAVE_JOBS = 65536
+WAVE_JOBS = 131072
 
 
 def pairs(rng, lengths, identity, indel):

@@ -14,6 +14,7 @@ from helpers import DELIM, concat, mutate, random_protein
 
 pytestmark = pytest.mark.gpu
 STALE, OVERFLOW = 1, 2
+GAP0, SUB, GAP1 = 0, 1, 2  # the oracle's edits
 
 
 def jobs_of(rng, lengths, identity, indel, at=None):
@@ -59,8 +60,9 @@ def on_host(q, d, job, cutoff):
 
 
 def by_oracle(q, d, job, cutoff, gap_open, gap_ext):
-    """The joined script's counts: the reverse side's operations in origin
-    order first, then the forward side's."""
+    """All fields but the flags: scores and ends of the two sides, and the
+    counts of the joined script, the reverse side's operations from its far
+    end on, then the forward side's."""
     m, nl = gz.blosum62()
     lead, qlen, hq, hd = (int(x) for x in job)
     s0, a0, b0, rev, _ = oracle_py.gapped_one_side(
@@ -69,7 +71,42 @@ def by_oracle(q, d, job, cutoff, gap_open, gap_ext):
     s1, a1, b1, fwd, _ = oracle_py.gapped_one_side(
         "oracle", q, lead + hq, qlen - hq, d, hd, DELIM, False, m, nl, gap_open, gap_ext, cutoff,
         traceback=True)
-    return s0 + s1, hq - 1 + a0, hd - 1 + b0, hq + a1, hd + b1, len(rev) + len(fwd)
+    script = rev[::-1] + fwd
+    qp, dp, mismatches, opens, extensions, prev = lead + hq - 1 + a0, hd - 1 + b0, 0, 0, 0, SUB
+    for op in script:
+        if op == SUB:
+            mismatches += q[qp] != d[dp]
+        elif op != prev:
+            opens += 1
+        else:
+            extensions += 1
+        qp, dp, prev = qp + (op != GAP0), dp + (op != GAP1), op
+    return (s0 + s1, hq - 1 + a0, hd - 1 + b0, hq + a1, hd + b1, len(script), int(mismatches),
+            opens, extensions)
+
+
+def off_the_waves(jobs):
+    """The same jobs, framed so that they take a lane each."""
+    part = jobs.copy()
+    part[:, 1] -= 1
+    return part
+
+
+def check_against_oracle(q, d, jobs, most, cutoff, gap_open, gap_ext):
+    """Every field against the oracle's script, and the flags against the
+    form of a lane per result; the share of results without a flag."""
+    out = build(q, d, jobs, most, cutoff, gap_open, gap_ext)
+    lanes = build(q, d, off_the_waves(jobs), most, cutoff, gap_open, gap_ext)
+    assert np.array_equal(out[:, 9], lanes[:, 9])
+    served = 0
+    for k, job in enumerate(jobs):
+        if out[k, 9]:
+            continue
+        served += 1
+        got = tuple(int(x) for x in out[k, :9].astype(np.int64))
+        want = by_oracle(q, d, job, cutoff, gap_open, gap_ext)
+        assert got == want, (k, job, got, want)
+    return served / len(jobs)
 
 
 # sides that end inside the 64-column window, at its edge and past it; bands
@@ -85,36 +122,42 @@ def test_waves_vs_host(cutoff, lengths, at):
     print("traceback waves: cutoff", cutoff, "lengths", lengths, "seed", at, flush=True)
     q, d, jobs, most = jobs_of(rng, np.repeat(lengths, 16), (0.3, 1.0), 0.05, at)
     out = build(q, d, jobs, most, cutoff)
-    stale = 0
     for k, job in enumerate(jobs):
         if out[k, 9] & OVERFLOW:  # 500 rows of bands past 130 columns fill the arena
-            assert job[1] * 230 > 1 << 16
+            assert cutoff == 120 and job[1] * 230 > 1 << 16
             continue
         host = on_host(q, d, job, cutoff)
         assert out[k, 9] == host[9], (k, job, out[k], host)
-        stale += int(host[9])
         if not host[9]:
             assert np.array_equal(out[k], host), (k, job, out[k], host)
-    print("  stale", stale, flush=True)
+
+
+@pytest.mark.parametrize("cutoff", [12, 20, 26])
+def test_stale_results_are_flagged(cutoff):
+    """Inputs on which a few paths read bytes that the extension did not
+    write: flagged where the host flags them, and where the form of a lane per
+    result does."""
+    rng = np.random.default_rng(cutoff)
+    print("traceback stale: cutoff", cutoff, flush=True)
+    q, d, jobs, most = jobs_of(rng, np.repeat((60, 150, 400), 130), (0.2, 1.0), 0.12)
+    out = build(q, d, jobs, most, cutoff)
+    host = np.array([on_host(q, d, job, cutoff) for job in jobs])
+    assert np.array_equal(out[:, 9], host[:, 9])
+    assert (host[:, 9] == STALE).sum() >= 2 and not (host[:, 9] & OVERFLOW).any()
+    fresh = host[:, 9] == 0
+    assert np.array_equal(out[fresh], host[fresh])
+    lanes = build(q, d, off_the_waves(jobs), most, cutoff)
+    assert np.array_equal(out[:, 9], lanes[:, 9]) and np.array_equal(out[fresh], lanes[fresh])
 
 
 @pytest.mark.parametrize("cutoff,gap_open,gap_ext", [
     (52, 11, 1), (60, 0, 3), (35, 8, 0), (52, 5, 2), (120, 30, 1), (10, 11, 1)])
 def test_waves_vs_oracle(cutoff, gap_open, gap_ext):
-    """Other gap costs: scores, both ends and the script's length."""
+    """Other gap costs: every field and the flags."""
     rng = np.random.default_rng(cutoff + 3 * gap_open)
     print("traceback waves: cutoff", cutoff, "gaps", gap_open, gap_ext, flush=True)
     q, d, jobs, most = jobs_of(rng, np.repeat((40, 63, 64, 130, 260), 20), (0.4, 1.0), 0.04)
-    out = build(q, d, jobs, most, cutoff, gap_open, gap_ext)
-    served = 0
-    for k, job in enumerate(jobs):
-        if out[k, 9]:
-            continue
-        served += 1
-        got = tuple(int(x) for x in out[k, :6].astype(np.int64))
-        want = by_oracle(q, d, job, cutoff, gap_open, gap_ext)
-        assert got == want, (k, job, got, want)
-    assert served > len(jobs) // 2
+    assert check_against_oracle(q, d, jobs, most, cutoff, gap_open, gap_ext) > 0.5
 
 
 @pytest.mark.parametrize("cutoff,gap_open,gap_ext", [
@@ -126,16 +169,7 @@ def test_wide_bands_vs_oracle(cutoff, gap_open, gap_ext):
     print("traceback wide bands: cutoff", cutoff, "gaps", gap_open, gap_ext, flush=True)
     q, d, jobs, most = jobs_of(rng, np.repeat((120, 200, 252, 255, 256, 260, 300), 12), (0.3, 1.0),
                                0.04, 0.0)
-    out = build(q, d, jobs, most, cutoff, gap_open, gap_ext)
-    served = 0
-    for k, job in enumerate(jobs):
-        if out[k, 9]:
-            continue
-        served += 1
-        got = tuple(int(x) for x in out[k, :6].astype(np.int64))
-        want = by_oracle(q, d, job, cutoff, gap_open, gap_ext)
-        assert got == want, (k, job, got, want)
-    assert served > len(jobs) // 2
+    assert check_against_oracle(q, d, jobs, most, cutoff, gap_open, gap_ext) > 0.5
 
 
 def test_more_jobs_than_waves():
@@ -191,7 +225,7 @@ def test_jobs_off_the_waves(lengths, n):
     full = build(q, d, jobs, most, 52)
     for every in (1, 40, n):
         part = jobs.copy()
-        part[::every, 1] -= 1  # the frame ends before the query's delimiter
+        part[::every] = off_the_waves(jobs[::every])
         assert np.array_equal(build(q, d, part, most, 52), full)
     large = build(q, d, jobs, most, 130)
     assert np.array_equal(large[:20], np.concatenate(
