@@ -640,10 +640,12 @@ __device__ void WaveSide(const WaveDpParams &P, const int8_t *sm, uint32_t q0, u
 //
 // Bound: the issue of a row's instructions (with the operations about 120,
 // against 90 without), then the path's dependent loads, a table entry and an
-// op per run of equal operations.  A call with its copies, against a lane per
-// result that walks the cells one by one with its op rows strided over the
-// chip's memory: 50,021 results of reads 5.9 -> 1.7 ms, 3,001 of proteins of
-// 100-500 residues 26 -> 1.0 ms.
+// op per run of equal operations.  A call with its copies and without
+// allocations, against a lane per result that walks the cells one by one with
+// its op rows strided over the chip's memory: 50,021 results of reads 5.9 ->
+// 1.34 ms (1.18 of it this kernel), 3,001 of proteins of 100-500 residues 26 ->
+// 0.64 ms; at cutoffs of 90 and 120 the latter 48 -> 0.92 and 63 -> 63 ms
+// (bands past 256 columns take a lane each).
 __global__ void __launch_bounds__(kTbWaveBlock)
     TracebackWaveKernel(WaveDpParams P, const TracebackJob *jobs, uint32_t n, uint32_t batch,
                         uint32_t *heads, const int *matrix, uint32_t nl, uint8_t *scratch,
