@@ -493,7 +493,7 @@ int Aligner::GappedRun(int slot, size_t ci, uint32_t nr, uint32_t nf, uint32_t *
     // the workspace for the largest bucket, allocated before any capture
     uint32_t most = 0;
     for (int b = 0; b < kLengthBuckets; ++b) most = std::max(most, bucket_off[b + 1] - bucket_off[b]);
-    if (gz_gapped_extender_reserve(gapped, most, &wrap) != GZ_OK) e = hipErrorUnknown;
+    if (!GappedReserveNow(gapped, most, s)) e = hipErrorUnknown;
   }
   if (bucketed) {
     // every query-length bucket with the configuration the tuner picks for

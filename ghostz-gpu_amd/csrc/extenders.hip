@@ -1481,17 +1481,20 @@ constexpr uint32_t kWideSlots = 256;
 constexpr uint32_t kWideSlotsMax = 16384;
 constexpr size_t kWideBudget = (size_t)8 << 30;
 
-// Lanes that a call of `size` jobs can use, and the ring's columns for them:
-// neither falls when the jobs or the longest query grow, so a ring of
-// RingColumns(size, wide) serves every call of up to `size` jobs and `wide`
-// columns, whichever form it takes.
-inline size_t RingLanes(size_t size) {
+// Waves of the global ring, where a wave takes a lane's slot.
+constexpr uint32_t kRingWaves = 4096;
+// Lanes that a call of `size` jobs can use out of `most` (kRingWaves or
+// kWideSlotsMax), and the ring's columns for them: neither falls when the jobs
+// or the longest query grow, so a ring of RingColumns(size, kWideSlotsMax, wide)
+// serves every call of up to `size` jobs and `wide` columns, whichever form it
+// takes.
+inline size_t RingLanes(size_t size, uint32_t most) {
   const size_t by_jobs = (size + 63) / 64 * 64;
-  return std::max<size_t>(kWideSlots, std::min<size_t>(kWideSlotsMax, by_jobs));
+  return std::max<size_t>(kWideSlots, std::min<size_t>(most, by_jobs));
 }
-inline size_t RingColumns(size_t size, uint32_t wide) {
+inline size_t RingColumns(size_t size, uint32_t most, uint32_t wide) {
   const size_t budget = kWideBudget / (sizeof(int2) + 1);
-  return std::max((size_t)kWideSlots * wide, std::min(budget, RingLanes(size) * wide));
+  return std::max((size_t)kWideSlots * wide, std::min(budget, RingLanes(size, most) * wide));
 }
 
 enum : int { kWaveAuto = 0, kWaveNever = 1, kWaveDirect = 2 };
@@ -1610,6 +1613,13 @@ static int RowColumns(const gz_gapped_extender_s *h) {
              : 0;
 }
 
+// Whether bands past the rings run one wave each, which is exact for cutoffs
+// below -kInitScore and non-negative gap costs, else one lane each.
+static bool RingByWaves(const gz_gapped_extender_s *h) {
+  return h->wave_mode != kWaveNever && h->cutoff < -kInitScore && h->gap_open >= 0 &&
+         h->gap_ext >= 0;
+}
+
 bool gz::GappedRunsRows(const gz_gapped_extender_s *h, size_t size) {
   return RowColumns(h) > 0 && size <= RowJobsFor(h->wide);
 }
@@ -1720,12 +1730,10 @@ static void GappedLaunch(gz_gapped_extender_t h, const GappedWork &w, const Gapp
     }
 #undef GZ_NARROW
   }
-  // bands past the 64-column ring: one wave per band when that is exact
-  // (the cutoff below -kInitScore and non-negative gap costs), else one lane
-  // per band; a wave takes a lane's slot of the global ring
-  const bool wave = h->wave_mode != kWaveNever && P.cutoff < -kInitScore && P.gap_open >= 0 &&
-                    P.gap_ext >= 0;
-  const dim3 wave_grid(std::min<uint32_t>(w.wide_slots, 4096u));
+  // bands past the 64-column ring: one wave or one lane per band; a wave takes
+  // a lane's slot of the global ring
+  const bool wave = RingByWaves(h);
+  const dim3 wave_grid(std::min<uint32_t>(w.wide_slots, kRingWaves));
   if (wave && h->wave_mode == kWaveDirect) {
     // the narrow ring's overflow straight to the waves
     hipLaunchKernelGGL((GappedWaveKernel<kReverse>), wave_grid, dim3(kWave), 0, s, P, h->matrix,
@@ -1780,8 +1788,8 @@ __global__ void ResetRunCountersKernel(uint32_t *counters, int all) {
 }
 
 // Allocates the handle's workspace for runs of up to `size` jobs (no-op
-// when it is large enough).
-static gz_status GappedReserve(gz_gapped_extender_t h, size_t size, hipStream_t s) {
+// when it is large enough), with the present settings or with any.
+static gz_status GappedReserve(gz_gapped_extender_t h, size_t size, bool any, hipStream_t s) {
   if (!h->counters) {
     GZ_HIP_CHECK(gz::Malloc(&h->counters, kRunCounters * sizeof(uint32_t)));
     hipLaunchKernelGGL(ResetRunCountersKernel, dim3(1), dim3(256), 0, s, h->counters, 1);
@@ -1797,7 +1805,8 @@ static gz_status GappedReserve(gz_gapped_extender_t h, size_t size, hipStream_t 
     GZ_HIP_CHECK(gz::Malloc(&h->overflow_list2, cap * sizeof(uint32_t)));
     h->overflow_capacity = cap;
   }
-  const size_t columns = RingColumns(size, h->wide);
+  const uint32_t most = any || !RingByWaves(h) ? kWideSlotsMax : kRingWaves;
+  const size_t columns = RingColumns(size, most, h->wide);
   if (h->ring_columns < columns) {
     if (h->wide_cells) GZ_HIP_CHECK(gz::Free(h->wide_cells));
     if (h->wide_codes) GZ_HIP_CHECK(gz::Free(h->wide_codes));
@@ -1811,6 +1820,10 @@ static gz_status GappedReserve(gz_gapped_extender_t h, size_t size, hipStream_t 
   return GZ_OK;
 }
 
+extern "C++" bool gz::GappedReserveNow(gz_gapped_extender_s *h, size_t size, hipStream_t s) {
+  return GappedReserve(h, size, false, s) == GZ_OK;
+}
+
 static gz_status GappedRun(gz_gapped_extender_t h, size_t size, int reverse,
                            uint32_t *d_q, uint32_t *d_d, int *d_scores,
                            uint32_t *d_cells, hipStream_t s, size_t wide_first = 0,
@@ -1819,13 +1832,15 @@ static gz_status GappedRun(gz_gapped_extender_t h, size_t size, int reverse,
              "gapped extender: queries, database and score parameters must be set");
   GZ_REQUIRE(wide_first <= size, "gapped extender: wide_first beyond the jobs");
   GZ_REQUIRE(size < (1ull << 31), "gapped extender: at most 2^31 - 1 jobs per call");
-  const gz_status rs = GappedReserve(h, size, s);
+  const gz_status rs = GappedReserve(h, size, false, s);
   if (rs != GZ_OK) return rs;
   // the overflow counts of this run start at zero; failures (counters[1])
   // are kept until gz_gapped_extender_failures reads them
   hipLaunchKernelGGL(ResetRunCountersKernel, dim3(1), dim3(256), 0, s, h->counters, 0);
   GZ_HIP_CHECK(hipGetLastError());
-  const size_t lanes = std::min(RingLanes(size), h->ring_columns / h->wide / 64 * 64);
+  const size_t lanes =
+      std::min(RingLanes(size, RingByWaves(h) ? kRingWaves : kWideSlotsMax),
+               h->ring_columns / h->wide / 64 * 64);
   const GappedWork w = {h->counters,   h->overflow_list, h->overflow_list2, h->wide_cells,
                         h->wide_codes, h->wide,          (uint32_t)lanes};
   h->failure_counter = h->counters + 1;
@@ -1968,7 +1983,7 @@ gz_status gz_gapped_extender_set_max_sequence_length(gz_gapped_extender_t h,
 
 gz_status gz_gapped_extender_reserve(gz_gapped_extender_t h, size_t size, gz_stream_t stream) {
   GZ_REQUIRE(h, "null handle");
-  return GappedReserve(h, size, S(stream));
+  return GappedReserve(h, size, true, S(stream));
 }
 
 gz_status gz_gapped_extender_set_persistent(gz_gapped_extender_t h, int persistent) {

@@ -17,6 +17,9 @@ namespace gz {
 // Whether a call of `size` jobs with the extender's present settings runs one
 // wave per job (extenders.hip): the first ring's settings then change nothing.
 bool GappedRunsRows(const gz_gapped_extender_s *h, size_t size);
+// The extender's workspace for calls of up to `size` jobs with its present
+// settings (gz_gapped_extender_reserve: with any); whether it could be had.
+bool GappedReserveNow(gz_gapped_extender_s *h, size_t size, hipStream_t s);
 
 // Stream capture and memory management exclude each other.  Freeing device
 // or pinned memory synchronizes the device, which a capture in flight on
