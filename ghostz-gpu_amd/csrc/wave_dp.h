@@ -102,13 +102,14 @@ constexpr int kWaveDpMargin = 16;
 // where lanes are the better form.  `wide`: the longest query side, as the
 // power of two of columns that it is given.
 //   * Two serve sides of up to 62 residues, which end inside the first
-//     window, and cutoffs that pay for few gaps, whose bands stay below 128
-//     columns and whose first row below 64.  The kernel for four
-//     keeps 84 registers instead of 47 and is 2 to 5% slower where two are
-//     enough (20,011 of 100-500 residues at cutoff 26, gaps 11/1: 309 us and 325;
-//     at 42 485 and 497); where they are not, jobs run again on the global
-//     ring (at 46 762 and 553, at 60 1,367 and 648; 3,001 of Pareto lengths
-//     at 60 70 ms and 19).
+//     window; sides of up to 126, which end inside the second, if their first
+//     row stays below 64 columns; and cutoffs that pay for few gaps, whose
+//     bands stay below 128.  The kernel for four keeps 84 registers instead of
+//     47 and is 2 to 5% slower where two are enough (20,011 of 100-500
+//     residues at cutoff 26, gaps 11/1: 309 us and 325; at 42 485 and 497;
+//     60,000 frames of 100 residues at 60 677 and 693); where they are not,
+//     jobs run again on the global ring (20,011 at 46 762 and 553, at 60 1,367
+//     and 648; 3,001 of Pareto lengths at 60 70 ms and 19).
 //   * Long sides whose bands outgrow 256 columns too pay for both forms, and
 //     the longest one's rows are the call's time: 3,001 of Pareto lengths at
 //     110 88 ms so and 68 on lanes, at 120 94 and 73, at 100 32 and 65; 3,000 of
@@ -120,6 +121,7 @@ inline int RowColumnsFor(int cutoff, int gap_open, int gap_ext, uint32_t wide) {
   if (wide <= 64 || cutoff < gap_init) return 2;
   if (gap_ext == 0) return 4;
   const int span = (cutoff - gap_init) / gap_ext + 1;  // columns that one gap can pass
+  if (wide <= 128 && span < kWave - 1) return 2;
   if (wide > 2048 && span * cutoff > 800 * gap_init) return 0;
   return span > 16 && 2 * cutoff > 7 * gap_init ? 4 : 2;
 }
